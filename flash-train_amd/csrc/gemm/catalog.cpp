@@ -73,8 +73,8 @@ constexpr VariantInfo kInfo[] = {
     {"Fp16MfmaGemm_128x128", 128, 128, 64, 256, 2, true, N, false, false, true, 0.4, FP16, 4096.0, 0.4},
     {"Fp16MfmaGemm_128x128_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.42, FP16, 4096.0, 0.3},
     {"Fp16MfmaGemm_64x64_Unaligned", 64, 64, 32, 256, 2, false, N, false, false, true, 0.08, FP16, 4096.0, 0.08},
-    {"Bf16MfmaGemm_256x256_Dma", 256, 256, 64, 256, 1, true, N, false, false, true, 0.66, BF16, 4096.0, 0.66},
-    {"Fp16MfmaGemm_256x256_Dma", 256, 256, 64, 256, 1, true, N, false, false, true, 0.66, FP16, 4096.0, 0.66},
+    {"Bf16MfmaGemm_256x256_Dma", 256, 256, 64, 512, 1, true, N, false, false, true, 0.66, BF16, 4096.0, 0.66},
+    {"Fp16MfmaGemm_256x256_Dma", 256, 256, 64, 512, 1, true, N, false, false, true, 0.66, FP16, 4096.0, 0.66},
     {"Bf16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, BF16, 4096.0, 0.45},
     {"Bf16MfmaGemm_128x128_Dma_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.55, BF16, 4096.0, 0.45},
     {"Fp16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, FP16, 4096.0, 0.45},

@@ -1,27 +1,26 @@
 // BF16 / FP16 tile kernels whose operands reach LDS by DMA
-// (global_load_lds_dwordx4) instead of through registers: 256x256 (plain and
-// grouped) and 128x128 (plain whole-k and split-k, grouped).
-// Device code only; the per-type translation units kernels_half_dma_*.hip
-// instantiate it.
+// (global_load_lds_dwordx4) instead of through registers: 128x128 (plain
+// whole-k and split-k, grouped) and 64x128 (split-k).  The 256x256 tile is
+// pingpong_tile.hpp's.  Device code only; the per-type translation units
+// kernels_half_dma_*.hip instantiate it.
 //
 // d = alpha * (a @ b) + beta * c, the same contract as the register-staged
 // tiles of half_tile.hpp (fp32 accumulation; c and d in fp32 or the input
 // type; with a null c the beta term is dropped).  Applicability, checked on
-// the host: k a multiple of 64 (no k tail: a DMA cannot zero-fill), a and b
-// 16-byte aligned with leading dimensions multiples of 8 elements and below
-// 2^23, c and d leading dimensions below 2^21 (32-bit offsets), contiguous
-// extents multiples of 8; m and n are free (edge tiles clamp their loads and
-// drop their out-of-matrix stores).
+// the host: a and b 16-byte aligned with leading dimensions multiples of 8
+// elements and below 2^23, c and d leading dimensions below 2^21 (32-bit
+// offsets), contiguous extents multiples of 8; m, n and k are free (edge
+// tiles clamp their loads and drop their out-of-matrix stores).
 //
-// Workgroup: 4 waves (one per SIMD), each a T/2 x T/2 block of the tile, as
-// (T/64) x (T/64) v_mfma_f32_32x32x16 blocks (4x4 at T = 256, 2x2 at 128):
+// Workgroup: 4 waves (one per SIMD), each a BM/2 x T/2 block of the tile, as
+// (BM/64) x (T/64) v_mfma_f32_32x32x16 blocks:
 //   A operand: lane l holds A[row l % 32][8 consecutive k]
 //   B operand: lane l holds B[the same 8 k][col l % 32]
 //   result   : lane l, register r holds D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32]
 // In k-step s (16 k) lane half h = l / 32 takes k 16 s + 8 h .. 16 s + 8 h + 7.
 //
-// Stage = 64 k of both operands, T x 64 x 2 bytes each; two LDS stages (128
-// KiB at T = 256, 64 KiB at 128).  One DMA instruction moves 64 lanes x 16
+// Stage = 64 k of both operands, BM x 64 and T x 64 elements; two LDS stages
+// (64 KiB at 128x128) or three.  One DMA instruction moves 64 lanes x 16
 // bytes into 1 KiB of LDS at M0 + 16 * lane, each lane from its own global
 // address, so a stage takes T/8 instructions per operand, T/32 per wave.
 // Each covers whole 128-byte lines:
@@ -40,17 +39,11 @@
 //     with X, and stage st + 1 has landed in Y;
 //   half 2: MFMAs on k 32..63 while reading k 0..31 of Y and issuing the
 //     DMA of stage st + 2 into X.
-// A DMA has one stage of MFMAs (2048 MFMA cycles per wave at T = 256) to land.  The
-// DMA is issued from inline assembly with M0 set in the same statement, so
-// the compiler's wait-count bookkeeping never sees it: every wait on it is
-// the explicit vmcnt in this file.  The compiler does not otherwise use M0
-// in this kernel (no LDS DMA builtins, no indexed register access: every
-// loop is unrolled).
-//
-// Measured on MI355X, same box and session, against the register-staged
-// 256x256 tile: bf16 8192^3 row-major a and b 848 against 991 us (every
-// orientation within 1%); MLP fwd 16384x14336x4096 1467 against 1748 us;
-// 4096^3 with c 125 against 158 us; MFMA busy 80-82%.
+// A DMA has one stage of MFMAs to land.  The DMA is issued from inline
+// assembly with M0 set in the same statement, so the compiler's wait-count
+// bookkeeping never sees it: every wait on it is the explicit vmcnt in this
+// file.  The compiler does not otherwise use M0 in this kernel (no LDS DMA
+// builtins, no indexed register access: every loop is unrolled).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -201,14 +194,12 @@ struct Operand {
 static __device__ __attribute__((aligned(256))) u16 dma_dummy[512];
 
 // Output tile `bid` of p (tile_of order), k split z when SPLIT; the whole workgroup calls it.
-// T: tile size (256: waves of 128x128, one workgroup per CU; 128: waves of 64x64, two per CU).
+// T: tile columns (128: waves of 64 columns, two workgroups per CU).
 // SPLIT: the workgroup reduces k range [z k_chunk, (z + 1) k_chunk) and stores its raw fp32 sums
 // to slice z of p.d (dense m x n); the reduction kernel forms d.
 // BM: tile rows (T by default; 64 with T = 128 for m of at most 64, row-major a only).
-// PF: stages of b to prefetch into L2 ahead of the stage being staged (0: none), for a b larger
-// than the MALL, whose stages otherwise arrive from HBM later than the DMA lead covers.
 // NB: stage buffers (2, or 3 for a ring in which each stage's DMAs run two stages ahead of its use).
-template <bool BF16, bool TA, bool TB, int T = 256, bool SPLIT = false, int BM = T, int PF = 0, int NB = 2>
+template <bool BF16, bool TA, bool TB, int T = 128, bool SPLIT = false, int BM = T, int NB = 2>
 // band: tile rows per band of the tile order (tile_of).
 __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int bid, int z = 0, int band = 8) {
     constexpr bool A_TR = TA, B_TR = !TB;
@@ -220,7 +211,7 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
     __shared__ __attribute__((aligned(1024))) u16 Bs0[kStageB];
     __shared__ __attribute__((aligned(1024))) u16 As1[kStageA];
     __shared__ __attribute__((aligned(1024))) u16 Bs1[kStageB];
-    static_assert(NB == 2 || (NB == 3 && PF == 0), "a three-buffer ring takes no prefetch");
+    static_assert(NB == 2 || NB == 3, "stage buffers");
     __shared__ __attribute__((aligned(1024))) u16 As2[NB > 2 ? kStageA : 8];
     __shared__ __attribute__((aligned(1024))) u16 Bs2[NB > 2 ? kStageB : 8];
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 31, h = lane >> 5;
@@ -250,36 +241,6 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
         opa.init(dma_dummy, 0, 0, BM, wave, lane);
         opb.init(dma_dummy, 0, 0, T, wave, lane);
     }
-    // L2 prefetch of b: one DMA per wave per stage, each lane touching one 128-byte line of the
-    // stage's b tile (256 lines at T = 256), into a 1 KiB sink per wave that nothing reads.  Lines
-    // past the matrix are clamped onto its last column (row-major b) or column (column-major b).
-    __shared__ __attribute__((aligned(1024))) u16 pf_sink[PF ? 4 * 512 : 8];
-    const unsigned lsink = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)pf_sink + wave * 1024;
-    unsigned pf_voff    = 0;
-    const char* pf_base = nullptr;
-    if constexpr (PF > 0) {
-        static_assert(T == 256, "prefetch lines cover a 256-column stage");
-        const int L = wave * 64 + lane;
-        if constexpr (B_TR) {  // row-major b: 64 k rows x T columns, T / 64 lines per row
-            constexpr int LPR = T / 64;
-            const int krow = L / LPR, line = L % LPR;
-            pf_voff = static_cast<unsigned>((krow * p.ldb + (min(n0 + 64 * line, N - 8) - n0)) * 2);
-            pf_base = reinterpret_cast<const char*>(pb + n0);
-        } else {  // column-major b: T columns of 64 k, one line each
-            pf_voff = static_cast<unsigned>((min(n0 + L, N - 1) - n0) * p.ldb * 2);
-            pf_base = reinterpret_cast<const char*>(pb + (size_t)n0 * p.ldb);
-        }
-        if (nst == 0) {  // every prefetch then reads stage 0 of the dummy
-            pf_voff = 0;
-            pf_base = reinterpret_cast<const char*>(dma_dummy);
-        }
-    }
-    auto prefetch = [&](int st) {
-        if constexpr (PF > 0) {
-            const size_t step = B_TR ? (size_t)kStageK * p.ldb * 2 : (size_t)kStageK * 2;
-            dma_1k(pf_voff, pf_base + (size_t)st * step, lsink);
-        }
-    };
     const unsigned la0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)As0;
     const unsigned lb0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)Bs0;
     const unsigned la1 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)As1;
@@ -370,8 +331,6 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
 #pragma unroll
                 for (int d = 0; d < ND; ++d)
                     if (((2 * d + 1) * NM) / (2 * ND) == t) dma_one(dma_st, d, la, lb);
-                // After the stage's last DMA: the prefetch is always the latest memory instruction.
-                if (PF > 0 && t == NM - 1) prefetch(min(dma_st + PF, last_st));
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -381,31 +340,26 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
         for (int r = 0; r < NR; ++r) read_one(ga, gb, As, Bs, hf, r);
     };
 
-    // Prologue: stages 0 and 1 in flight (ND DMAs per wave each), with prefetch stages 2 .. PF + 1
-    // too; wait for stage 0.  Each wait below then leaves exactly one instruction pending, the
-    // latest prefetch (memory instructions complete in issue order for the counter).  With no whole
+    // Prologue: the first NB stages in flight (ND DMAs per wave each); wait for stage 0.  With no whole
     // stage it reads the dummy.
 #pragma unroll
     for (int d = 0; d < ND; ++d) dma_one(0, d, la0, lb0);
-#pragma unroll
-    for (int i = 2; i <= PF; ++i) prefetch(min(i, last_st));
     const int st1 = min(1, last_st);
 #pragma unroll
     for (int d = 0; d < ND; ++d) dma_one(st1, d, la1, lb1);
-    prefetch(min(1 + PF, last_st));
     if constexpr (NB == 3) {
         const int st2 = min(2, last_st);
 #pragma unroll
         for (int d = 0; d < ND; ++d) dma_one(st2, d, la2, lb2);
     }
-    static_assert((NB - 1) * ND + PF <= 63, "the wait count field holds 63");
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NB - 1) * ND + PF) : "memory");
+    static_assert((NB - 1) * ND <= 63, "the wait count field holds 63");
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NB - 1) * ND) : "memory");
     read_half(fa0, fb0, As0, Bs0, 0);
 
     // Stages past the last reload the last one (harmless: nothing reads them).
 #define FT_DMA_PHASE(XA, XB, YA, YB, LXA, LXB, ST)                               \
     run_half(fa0, fb0, fa1, fb1, XA, XB, 1, std::false_type{}, 0, 0u, 0u);                          \
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PF > 0 ? 1 : 0) : "memory"); \
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); \
     run_half(fa1, fb1, fa0, fb0, YA, YB, 0, std::true_type{}, min((ST) + 2, last_st), LXA, LXB);
     // Ring: the wait for the next stage leaves the one after it in flight, and the freed buffer
     // takes the stage three ahead.
@@ -461,7 +415,7 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
     // Epilogue through buffer loads and stores relative to the tile's corner.  The byte offset of
     // an element splits into a per-lane part (4 h rows and lane column li) in the VGPR offset and
     // a wave-uniform part (block, register) in the scalar offset.  An element outside the matrix
-    // (edge tiles: a grouped GEMM's last rows, any m or n not a multiple of 256) gets the lane
+    // (edge tiles: a grouped GEMM's last rows, any m or n not a multiple of the tile) gets the lane
     // offset 2^31, past the buffer's size (at most 2^31 - 1 bytes), so its c load returns 0 and
     // its store is dropped by the hardware range check: no branches, one copy for whole and edge
     // tiles.  ldc, ldd below 2^21 (checked on the host) keep every sum below 2^32.
@@ -540,11 +494,6 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
     }
 }
 
-template <bool BF16, bool TA, bool TB, int PF = 0>
-__global__ __launch_bounds__(256, 1) void half_gemm_dma(HalfGemmParams p) {
-    half_gemm_dma_tile<BF16, TA, TB, 256, false, 256, PF>(p, blockIdx.x);
-}
-
 // 128x128 tiles, two workgroups per CU, whole-k or split-k.  Split-k workgroups are renumbered so
 // each XCD runs whole k splits (hardware ids go to the XCDs in turn, x fastest).
 template <bool BF16, bool TA, bool TB, bool SPLIT>
@@ -579,7 +528,7 @@ __global__ __launch_bounds__(256, 2) void half_gemm_dma64x128(HalfGemmParams p) 
         const int t   = w - z * tiles, per = tiles >> 3;
         bid           = t < (per << 3) ? ((t % per) << 3) + t / per : t;
     }
-    half_gemm_dma_tile<BF16, false, TB, 128, true, 64, 0, 3>(p, bid, z);
+    half_gemm_dma_tile<BF16, false, TB, 128, true, 64, 3>(p, bid, z);
 }
 
 // Grouped GEMM over a device table of per-group parameters: the workgroup's
@@ -587,8 +536,8 @@ __global__ __launch_bounds__(256, 2) void half_gemm_dma64x128(HalfGemmParams p) 
 // are multiples of 8, so the group-local id keeps the hardware id's XCD;
 // ids past the group's tiles are padding and exit at once (before any
 // barrier, the whole workgroup).
-template <bool BF16, bool TA, bool TB, int T = 256, int PF = 0>
-__global__ __launch_bounds__(256, 256 / T) void grouped_half_gemm_dma(GroupedHalfArgs g) {
+template <bool BF16, bool TA, bool TB>
+__global__ __launch_bounds__(256, 2) void grouped_half_gemm_dma(GroupedHalfArgs g) {
     const int bid = blockIdx.x;
     int lo = 0, hi = g.groups - 1;
     while (lo < hi) {
@@ -603,21 +552,18 @@ __global__ __launch_bounds__(256, 256 / T) void grouped_half_gemm_dma(GroupedHal
     if (local >= p.tiles_m * p.tiles_n) return;
     // One band per group when the group has at most kGroupBand tile rows: each group has a b of its
     // own, which bands of 8 rows fetched once per band (8 MoE experts of 4 to 13 tile rows: 1.5x
-    // the b bytes of one band per expert).  With the L2 prefetch of b those re-reads are cheap and
-    // bands of 8 rows, which re-read less of a, are faster (8 experts, 940 MB of weights: 1.638
-    // against 1.662 ms).
-    const int band = PF > 0 ? 8 : p.tiles_m <= kGroupBand ? p.tiles_m : 8;
-    half_gemm_dma_tile<BF16, TA, TB, T, false, T, PF>(p, local, 0, band);
+    // the b bytes of one band per expert).
+    const int band = p.tiles_m <= kGroupBand ? p.tiles_m : 8;
+    half_gemm_dma_tile<BF16, TA, TB, 128>(p, local, 0, band);
 }
 
-// Kernel for one input type, tile size and operand orientation (ta: column-major a, tb:
-// column-major b).
-template <bool BF16, int T = 256, int PF = 0>
+// Kernel for one input type and operand orientation (ta: column-major a, tb: column-major b).
+template <bool BF16>
 const void* groupedDmaKernel(bool ta, bool tb) {
-    if (ta) return tb ? reinterpret_cast<const void*>(&grouped_half_gemm_dma<BF16, true, true, T, PF>)
-                      : reinterpret_cast<const void*>(&grouped_half_gemm_dma<BF16, true, false, T, PF>);
-    return tb ? reinterpret_cast<const void*>(&grouped_half_gemm_dma<BF16, false, true, T, PF>)
-              : reinterpret_cast<const void*>(&grouped_half_gemm_dma<BF16, false, false, T, PF>);
+    if (ta) return tb ? reinterpret_cast<const void*>(&grouped_half_gemm_dma<BF16, true, true>)
+                      : reinterpret_cast<const void*>(&grouped_half_gemm_dma<BF16, true, false>);
+    return tb ? reinterpret_cast<const void*>(&grouped_half_gemm_dma<BF16, false, true>)
+              : reinterpret_cast<const void*>(&grouped_half_gemm_dma<BF16, false, false>);
 }
 template <bool BF16, bool SPLIT>
 const void* dma128Kernel(bool ta, bool tb) {
@@ -632,19 +578,4 @@ const void* dma64x128Kernel(bool ta, bool tb) {
     return tb ? reinterpret_cast<const void*>(&half_gemm_dma64x128<BF16, true>)
               : reinterpret_cast<const void*>(&half_gemm_dma64x128<BF16, false>);
 }
-// Stages of b a large-b launch prefetches ahead (measured: 2048x114688x4096 bf16 1508-1512 us at 4,
-// 1517-1530 at 2, 1620-1633 without).
-constexpr int kLargeBPrefetch = 4;
-template <bool BF16, int PF = 0>
-const void* dmaKernelFor(bool ta, bool tb) {
-    if (ta) return tb ? reinterpret_cast<const void*>(&half_gemm_dma<BF16, true, true, PF>)
-                      : reinterpret_cast<const void*>(&half_gemm_dma<BF16, true, false, PF>);
-    return tb ? reinterpret_cast<const void*>(&half_gemm_dma<BF16, false, true, PF>)
-              : reinterpret_cast<const void*>(&half_gemm_dma<BF16, false, false, PF>);
-}
-template <bool BF16>
-const void* dmaKernel(bool ta, bool tb, bool prefetch_b) {
-    return prefetch_b ? dmaKernelFor<BF16, kLargeBPrefetch>(ta, tb) : dmaKernelFor<BF16>(ta, tb);
-}
-
 }  // namespace ftrain::gemm::ddev

@@ -1,15 +1,15 @@
-// BF16 256x256 tiles with LDS staging by DMA, every operand orientation (see gemm/dma_tile.hpp).
+// BF16 tiles with LDS staging by DMA, every operand orientation: 256x256 (gemm/pingpong_tile.hpp),
+// 128x128 and 64x128 (gemm/dma_tile.hpp).
 #include "dma_tile.hpp"
+#include "pingpong_tile.hpp"
 
 namespace ftrain::gemm {
 
-const void* dmaKernelBf16(bool ta, bool tb, bool prefetch_b) { return ddev::dmaKernel<true>(ta, tb, prefetch_b); }
+const void* dmaKernelBf16(bool ta, bool tb) { return ppdev::ppKernel<true>(ta, tb); }
 
-const void* groupedDmaKernelBf16(bool ta, bool tb, bool prefetch_b) {
-    return prefetch_b ? ddev::groupedDmaKernel<true, 256, ddev::kLargeBPrefetch>(ta, tb) : ddev::groupedDmaKernel<true>(ta, tb);
-}
+const void* groupedDmaKernelBf16(bool ta, bool tb) { return ppdev::groupedPpKernel<true>(ta, tb); }
 
-const void* groupedDma128KernelBf16(bool ta, bool tb) { return ddev::groupedDmaKernel<true, 128>(ta, tb); }
+const void* groupedDma128KernelBf16(bool ta, bool tb) { return ddev::groupedDmaKernel<true>(ta, tb); }
 
 const void* dma64x128KernelBf16(bool ta, bool tb) { return ddev::dma64x128Kernel<true>(ta, tb); }
 
