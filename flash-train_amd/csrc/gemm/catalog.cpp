@@ -75,10 +75,10 @@ constexpr VariantInfo kInfo[] = {
     {"Fp16MfmaGemm_64x64_Unaligned", 64, 64, 32, 256, 2, false, N, false, false, true, 0.08, FP16, 4096.0, 0.08},
     {"Bf16MfmaGemm_256x256_Dma", 256, 256, 64, 512, 1, true, N, false, false, true, 0.66, BF16, 4096.0, 0.66},
     {"Fp16MfmaGemm_256x256_Dma", 256, 256, 64, 512, 1, true, N, false, false, true, 0.66, FP16, 4096.0, 0.66},
-    {"Bf16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, BF16, 4096.0, 0.45},
-    {"Bf16MfmaGemm_128x128_Dma_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.55, BF16, 4096.0, 0.45},
-    {"Fp16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, FP16, 4096.0, 0.45},
-    {"Fp16MfmaGemm_128x128_Dma_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.55, FP16, 4096.0, 0.45},
+    {"Bf16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, BF16, 4096.0, 0.65},
+    {"Bf16MfmaGemm_128x128_Dma_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.55, BF16, 4096.0, 0.65},
+    {"Fp16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, FP16, 4096.0, 0.65},
+    {"Fp16MfmaGemm_128x128_Dma_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.55, FP16, 4096.0, 0.65},
     // Applicable to m of at most 64 only.  The low single-workgroup figure makes the model spread
     // such a problem over 8 splits (one workgroup per CU), as measured (64x4096x4096: 4 splits
     // leave half the CUs idle).

@@ -189,6 +189,15 @@ struct Operand {
     }
 };
 
+// f(integral_constant<I>) for I in [FIRST, LAST).
+template <int FIRST, int LAST, class F>
+__device__ __forceinline__ void each(F&& f) {
+    if constexpr (FIRST < LAST) {
+        f(std::integral_constant<int, FIRST>{});
+        each<FIRST + 1, LAST>(f);
+    }
+}
+
 // What the DMA pipeline reads when k holds no whole stage (its data is discarded): operands
 // initialised on it with a leading dimension of 0 keep every lane's offset within 512 bytes.
 static __device__ __attribute__((aligned(256))) u16 dma_dummy[512];
@@ -198,7 +207,7 @@ static __device__ __attribute__((aligned(256))) u16 dma_dummy[512];
 // SPLIT: the workgroup reduces k range [z k_chunk, (z + 1) k_chunk) and stores its raw fp32 sums
 // to slice z of p.d (dense m x n); the reduction kernel forms d.
 // BM: tile rows (T by default; 64 with T = 128 for m of at most 64, row-major a only).
-// NB: stage buffers (2, or 3 for a ring in which each stage's DMAs run two stages ahead of its use).
+// NB: stage buffers; a stage's DMAs run NB - 1 stages ahead of its use.
 template <bool BF16, bool TA, bool TB, int T = 128, bool SPLIT = false, int BM = T, int NB = 2>
 // band: tile rows per band of the tile order (tile_of).
 __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int bid, int z = 0, int band = 8) {
@@ -207,13 +216,8 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
     constexpr int NBM = BM / 64, NBN = T / 64;  // 32x32 blocks per wave row / column
     constexpr int NDA = BM / 32, NDB = T / 32;  // DMAs per wave per stage: A, B
     constexpr int kStageA = BM * kStageK, kStageB = T * kStageK;  // one operand, one stage
-    __shared__ __attribute__((aligned(1024))) u16 As0[kStageA];
-    __shared__ __attribute__((aligned(1024))) u16 Bs0[kStageB];
-    __shared__ __attribute__((aligned(1024))) u16 As1[kStageA];
-    __shared__ __attribute__((aligned(1024))) u16 Bs1[kStageB];
-    static_assert(NB == 2 || NB == 3, "stage buffers");
-    __shared__ __attribute__((aligned(1024))) u16 As2[NB > 2 ? kStageA : 8];
-    __shared__ __attribute__((aligned(1024))) u16 Bs2[NB > 2 ? kStageB : 8];
+    __shared__ __attribute__((aligned(1024))) u16 As[NB][kStageA];
+    __shared__ __attribute__((aligned(1024))) u16 Bs[NB][kStageB];
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wrow = (wave >> 1) * (BM / 2), wcol = (wave & 1) * (T / 2);
@@ -241,12 +245,8 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
         opa.init(dma_dummy, 0, 0, BM, wave, lane);
         opb.init(dma_dummy, 0, 0, T, wave, lane);
     }
-    const unsigned la0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)As0;
-    const unsigned lb0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)Bs0;
-    const unsigned la1 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)As1;
-    const unsigned lb1 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)Bs1;
-    const unsigned la2 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)As2;
-    const unsigned lb2 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)Bs2;
+    const unsigned la = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)&As[0][0];
+    const unsigned lb = (unsigned)(uintptr_t)(__attribute__((address_space(3))) u16*)&Bs[0][0];
 
     // Operand of k-step ks (0..3 in the stage) for rows (or columns) x .. x + 31.
     const int tr_k = (lane & 15) >> 2, tr_x = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
@@ -280,17 +280,18 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
     constexpr int NM = 2 * NBM * NBN;  // MFMAs per half stage
     constexpr int ND = NDA + NDB;      // DMAs per wave per stage
     // DMA d (0 .. ND - 1) of a stage: A and B alternate while both have some left.
-    auto dma_one = [&](int st, int d, unsigned la, unsigned lb) {
+    auto dma_one = [&](int st, int d, int buf) {
         constexpr int PAIRS = NDA < NDB ? NDA : NDB;
+        const unsigned da = la + buf * kStageA * 2, db = lb + buf * kStageB * 2;
         if (d < 2 * PAIRS) {
             if (d & 1)
-                opb.dma(st, d >> 1, lb, wave);
+                opb.dma(st, d >> 1, db, wave);
             else
-                opa.dma(st, d >> 1, la, wave);
+                opa.dma(st, d >> 1, da, wave);
         } else if (NDA > NDB) {
-            opa.dma(st, d - PAIRS, la, wave);
+            opa.dma(st, d - PAIRS, da, wave);
         } else {
-            opb.dma(st, d - PAIRS, lb, wave);
+            opb.dma(st, d - PAIRS, db, wave);
         }
     };
     // LDS read r (0 .. NR-1) of half `hf`, ordered k-step major (A then B within a k-step), into (ga, gb).
@@ -316,10 +317,10 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
         }
     };
     // NM MFMAs on (fa, fb) (k-step major, then block row, block column); the NR reads of half hf
-    // of (As, Bs) into (ga, gb) and, with a true with_dma, the ND DMAs of stage dma_st into (la,
-    // lb) (A and B alternating) are spread between them in a fixed order.
+    // of (As, Bs) into (ga, gb) and, with a true with_dma, the ND DMAs of stage dma_st into buffer
+    // buf (A and B alternating) are spread between them in a fixed order.
     auto run_half = [&](u32x4 (&fa)[2][NBM], u32x4 (&fb)[2][NBN], u32x4 (&ga)[2][NBM], u32x4 (&gb)[2][NBN],
-                        const u16* As, const u16* Bs, int hf, auto with_dma, int dma_st, unsigned la, unsigned lb) {
+                        const u16* As, const u16* Bs, int hf, auto with_dma, int dma_st, int buf) {
 #pragma unroll
         for (int t = 0; t < NM; ++t) {
             const int s = t / (NBM * NBN), bi = (t / NBN) % NBM, bj = t % NBN;
@@ -330,7 +331,7 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
             if constexpr (decltype(with_dma)::value) {
 #pragma unroll
                 for (int d = 0; d < ND; ++d)
-                    if (((2 * d + 1) * NM) / (2 * ND) == t) dma_one(dma_st, d, la, lb);
+                    if (((2 * d + 1) * NM) / (2 * ND) == t) dma_one(dma_st, d, buf);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -343,56 +344,29 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
     // Prologue: the first NB stages in flight (ND DMAs per wave each); wait for stage 0.  With no whole
     // stage it reads the dummy.
 #pragma unroll
-    for (int d = 0; d < ND; ++d) dma_one(0, d, la0, lb0);
-    const int st1 = min(1, last_st);
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
-    for (int d = 0; d < ND; ++d) dma_one(st1, d, la1, lb1);
-    if constexpr (NB == 3) {
-        const int st2 = min(2, last_st);
-#pragma unroll
-        for (int d = 0; d < ND; ++d) dma_one(st2, d, la2, lb2);
-    }
+        for (int d = 0; d < ND; ++d) dma_one(min(i, last_st), d, i);
     static_assert((NB - 1) * ND <= 63, "the wait count field holds 63");
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NB - 1) * ND) : "memory");
-    read_half(fa0, fb0, As0, Bs0, 0);
+    read_half(fa0, fb0, As[0], Bs[0], 0);
 
-    // Stages past the last reload the last one (harmless: nothing reads them).
-#define FT_DMA_PHASE(XA, XB, YA, YB, LXA, LXB, ST)                               \
-    run_half(fa0, fb0, fa1, fb1, XA, XB, 1, std::false_type{}, 0, 0u, 0u);                          \
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); \
-    run_half(fa1, fb1, fa0, fb0, YA, YB, 0, std::true_type{}, min((ST) + 2, last_st), LXA, LXB);
-    // Ring: the wait for the next stage leaves the one after it in flight, and the freed buffer
-    // takes the stage three ahead.
-#define FT_RING_PHASE(XA, XB, YA, YB, LXA, LXB, ST)                                                  \
-    run_half(fa0, fb0, fa1, fb1, XA, XB, 1, std::false_type{}, 0, 0u, 0u);                          \
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(ND) : "memory");   \
-    run_half(fa1, fb1, fa0, fb0, YA, YB, 0, std::true_type{}, min((ST) + 3, last_st), LXA, LXB);
+    // Stage st in buffer X (a constant): the wait for the next stage leaves the NB - 2 after it in
+    // flight, and the freed buffer takes the stage NB ahead.  Stages past the last reload the last
+    // one (harmless: nothing reads them).
+    auto phase = [&](auto x_tag, int st) {
+        constexpr int X = decltype(x_tag)::value, Y = (X + 1) % NB;
+        run_half(fa0, fb0, fa1, fb1, As[X], Bs[X], 1, std::false_type{}, 0, 0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NB - 2) * ND) : "memory");
+        run_half(fa1, fb1, fa0, fb0, As[Y], Bs[Y], 0, std::true_type{}, min(st + NB, last_st), X);
+    };
     int st = 0;
-    if constexpr (NB == 2) {
-        for (; st + 1 < nst; st += 2) {
-            FT_DMA_PHASE(As0, Bs0, As1, Bs1, la0, lb0, st)
-            FT_DMA_PHASE(As1, Bs1, As0, Bs0, la1, lb1, st + 1)
-        }
-        // An odd stage count ends with one more stage in buffer 0 (a separate copy: leaving the
-        // loop between its two phases costs the register allocator the fragment double buffer).
-        if (st < nst) {
-            FT_DMA_PHASE(As0, Bs0, As1, Bs1, la0, lb0, st)
-        }
-    } else {
-        for (; st + 2 < nst; st += 3) {
-            FT_RING_PHASE(As0, Bs0, As1, Bs1, la0, lb0, st)
-            FT_RING_PHASE(As1, Bs1, As2, Bs2, la1, lb1, st + 1)
-            FT_RING_PHASE(As2, Bs2, As0, Bs0, la2, lb2, st + 2)
-        }
-        if (st < nst) {
-            FT_RING_PHASE(As0, Bs0, As1, Bs1, la0, lb0, st)
-        }
-        if (st + 1 < nst) {
-            FT_RING_PHASE(As1, Bs1, As2, Bs2, la1, lb1, st + 1)
-        }
-    }
-#undef FT_RING_PHASE
-#undef FT_DMA_PHASE
+    for (; st + NB - 1 < nst; st += NB) each<0, NB>([&](auto x) { phase(x, st + decltype(x)::value); });
+    // The remaining stages (separate copies: leaving the loop between its phases costs the register
+    // allocator the fragment double buffer).
+    each<0, NB - 1>([&](auto x) {
+        if (st + decltype(x)::value < nst) phase(x, st + decltype(x)::value);
+    });
     // The workgroup's LDS must not be released with a DMA still writing it.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
@@ -403,13 +377,13 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
         opa.init(pa, p.lda, m0, M, wave, lane);
         opb.init(pb, p.ldb, n0, N, wave, lane);
 #pragma unroll
-        for (int j = 0; j < NDA; ++j) opa.fill(nst, j, As0, wave, lane, k_tail);
+        for (int j = 0; j < NDA; ++j) opa.fill(nst, j, As[0], wave, lane, k_tail);
 #pragma unroll
-        for (int j = 0; j < NDB; ++j) opb.fill(nst, j, Bs0, wave, lane, k_tail);
+        for (int j = 0; j < NDB; ++j) opb.fill(nst, j, Bs[0], wave, lane, k_tail);
         __syncthreads();
-        read_half(fa0, fb0, As0, Bs0, 0);
-        run_half(fa0, fb0, fa1, fb1, As0, Bs0, 1, std::false_type{}, 0, 0u, 0u);
-        run_half(fa1, fb1, fa0, fb0, As0, Bs0, 0, std::false_type{}, 0, 0u, 0u);
+        read_half(fa0, fb0, As[0], Bs[0], 0);
+        run_half(fa0, fb0, fa1, fb1, As[0], Bs[0], 1, std::false_type{}, 0, 0);
+        run_half(fa1, fb1, fa0, fb0, As[0], Bs[0], 0, std::false_type{}, 0, 0);
     }
 
     // Epilogue through buffer loads and stores relative to the tile's corner.  The byte offset of
@@ -494,10 +468,15 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
     }
 }
 
-// 128x128 tiles, two workgroups per CU, whole-k or split-k.  Split-k workgroups are renumbered so
-// each XCD runs whole k splits (hardware ids go to the XCDs in turn, x fastest).
-template <bool BF16, bool TA, bool TB, bool SPLIT>
-__global__ __launch_bounds__(256, 2) void half_gemm_dma128(HalfGemmParams p) {
+// 128x128 tiles, whole-k or split-k.  Split-k workgroups are renumbered so each XCD runs whole k
+// splits (hardware ids go to the XCDs in turn, x fastest).
+// SOLO: for a launch of no more workgroups than CUs.  Two stage buffers (64 KiB, two workgroups per
+// CU) leave a lone workgroup waiting for its one stage in flight: 0.61 us per 64-k stage against
+// 0.21 us of MFMAs.  Three (96 KiB) keep two in flight, which is all it can use (four measured the
+// same): bf16 whole-k 512x4096x4096 41.9 -> 26.0 us, 1024x4096x4096 40.8 -> 32.1, 2048^3 25.3 -> 19.1;
+// with more workgroups than CUs two per CU stay ahead (2048x4096x4096, 512 tiles, 58.9 against 62.7).
+template <bool BF16, bool TA, bool TB, bool SPLIT, bool SOLO>
+__global__ __launch_bounds__(256, SOLO ? 1 : 2) void half_gemm_dma128(HalfGemmParams p) {
     int bid = blockIdx.x, z = blockIdx.z;
     if constexpr (SPLIT) {
         const int tiles = gridDim.x, total = tiles * gridDim.z;
@@ -509,7 +488,7 @@ __global__ __launch_bounds__(256, 2) void half_gemm_dma128(HalfGemmParams p) {
             bid           = t < (per << 3) ? ((t % per) << 3) + t / per : t;
         }
     }
-    half_gemm_dma_tile<BF16, TA, TB, 128, SPLIT>(p, bid, z);
+    half_gemm_dma_tile<BF16, TA, TB, 128, SPLIT, 128, SOLO ? 3 : 2>(p, bid, z);
 }
 
 // 64x128 split-k tiles for m of at most 64 (a 128-row tile would stage and multiply 64 rows of
@@ -565,12 +544,17 @@ const void* groupedDmaKernel(bool ta, bool tb) {
     return tb ? reinterpret_cast<const void*>(&grouped_half_gemm_dma<BF16, false, true>)
               : reinterpret_cast<const void*>(&grouped_half_gemm_dma<BF16, false, false>);
 }
-template <bool BF16, bool SPLIT>
-const void* dma128Kernel(bool ta, bool tb) {
-    if (ta) return tb ? reinterpret_cast<const void*>(&half_gemm_dma128<BF16, true, true, SPLIT>)
-                      : reinterpret_cast<const void*>(&half_gemm_dma128<BF16, true, false, SPLIT>);
-    return tb ? reinterpret_cast<const void*>(&half_gemm_dma128<BF16, false, true, SPLIT>)
-              : reinterpret_cast<const void*>(&half_gemm_dma128<BF16, false, false, SPLIT>);
+template <bool BF16, bool SPLIT, bool SOLO>
+const void* dma128KernelFor(bool ta, bool tb) {
+    if (ta) return tb ? reinterpret_cast<const void*>(&half_gemm_dma128<BF16, true, true, SPLIT, SOLO>)
+                      : reinterpret_cast<const void*>(&half_gemm_dma128<BF16, true, false, SPLIT, SOLO>);
+    return tb ? reinterpret_cast<const void*>(&half_gemm_dma128<BF16, false, true, SPLIT, SOLO>)
+              : reinterpret_cast<const void*>(&half_gemm_dma128<BF16, false, false, SPLIT, SOLO>);
+}
+template <bool BF16>
+const void* dma128Kernel(bool ta, bool tb, bool split, bool solo) {
+    if (split) return solo ? dma128KernelFor<BF16, true, true>(ta, tb) : dma128KernelFor<BF16, true, false>(ta, tb);
+    return solo ? dma128KernelFor<BF16, false, true>(ta, tb) : dma128KernelFor<BF16, false, false>(ta, tb);
 }
 template <bool BF16>
 const void* dma64x128Kernel(bool ta, bool tb) {

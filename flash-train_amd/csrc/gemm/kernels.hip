@@ -411,7 +411,7 @@ const void* gemvKernel(Variant v, int m, bool ta, int& threads) {
     return ta ? reinterpret_cast<const void*>(&gemv_pass<8, 2, 8, true>) : reinterpret_cast<const void*>(&gemv_pass<8, 2, 8, false>);
 }
 
-const void* kernelFor(Variant v, bool ta, bool tb) {
+const void* kernelFor(Variant v, bool ta, bool tb, bool solo) {
     if (info(v).gemv && info(v).split == SplitKind::kNone) {
         if (tb) return nullptr;
         int threads = 0;
@@ -435,9 +435,9 @@ const void* kernelFor(Variant v, bool ta, bool tb) {
     if (v == Variant::kBf16MfmaDma256x256) return dmaKernelBf16(ta, tb);
     if (v == Variant::kFp16MfmaDma256x256) return dmaKernelFp16(ta, tb);
     if (v == Variant::kBf16MfmaDma128x128 || v == Variant::kBf16MfmaDma128x128S)
-        return dma128KernelBf16(ta, tb, v == Variant::kBf16MfmaDma128x128S);
+        return dma128KernelBf16(ta, tb, v == Variant::kBf16MfmaDma128x128S, solo);
     if (v == Variant::kFp16MfmaDma128x128 || v == Variant::kFp16MfmaDma128x128S)
-        return dma128KernelFp16(ta, tb, v == Variant::kFp16MfmaDma128x128S);
+        return dma128KernelFp16(ta, tb, v == Variant::kFp16MfmaDma128x128S, solo);
     if (v == Variant::kBf16MfmaDma64x128S) return dma64x128KernelBf16(ta, tb);
     if (v == Variant::kFp16MfmaDma64x128S) return dma64x128KernelFp16(ta, tb);
     if (ta || tb) {

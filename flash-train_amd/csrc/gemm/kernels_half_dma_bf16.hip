@@ -13,8 +13,8 @@ const void* groupedDma128KernelBf16(bool ta, bool tb) { return ddev::groupedDmaK
 
 const void* dma64x128KernelBf16(bool ta, bool tb) { return ddev::dma64x128Kernel<true>(ta, tb); }
 
-const void* dma128KernelBf16(bool ta, bool tb, bool split) {
-    return split ? ddev::dma128Kernel<true, true>(ta, tb) : ddev::dma128Kernel<true, false>(ta, tb);
+const void* dma128KernelBf16(bool ta, bool tb, bool split, bool solo) {
+    return ddev::dma128Kernel<true>(ta, tb, split, solo);
 }
 
 }  // namespace ftrain::gemm

@@ -13,8 +13,8 @@ const void* groupedDma128KernelFp16(bool ta, bool tb) { return ddev::groupedDmaK
 
 const void* dma64x128KernelFp16(bool ta, bool tb) { return ddev::dma64x128Kernel<false>(ta, tb); }
 
-const void* dma128KernelFp16(bool ta, bool tb, bool split) {
-    return split ? ddev::dma128Kernel<false, true>(ta, tb) : ddev::dma128Kernel<false, false>(ta, tb);
+const void* dma128KernelFp16(bool ta, bool tb, bool split, bool solo) {
+    return ddev::dma128Kernel<false>(ta, tb, split, solo);
 }
 
 }  // namespace ftrain::gemm

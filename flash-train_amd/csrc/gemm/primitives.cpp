@@ -243,6 +243,7 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
             params_.tiles_m = half_params_.tiles_m = int32_t(ceilDiv(s.m, info_->bm));
             params_.tiles_n = half_params_.tiles_n = int32_t(ceilDiv(s.n, info_->bn));
             grid_           = dim3(uint32_t(params_.tiles_m) * uint32_t(params_.tiles_n), 1, splits);
+            kernel_         = gemm::kernelFor(v_, g.ta, g.tb, uint64_t(grid_.x) * splits <= uint64_t(cus));
         }
         const uint64_t count = s.m * s.n;
         if (info_->split == SplitKind::kFused) {

@@ -258,7 +258,9 @@ const VariantInfo& info(Variant v);
 // kernelFor: the variant's kernel for a column-major (ta) or row-major a and
 // a column-major (tb) or row-major b; null when that layout is not
 // instantiated for the variant (see VariantInfo::layouts).
-const void* kernelFor(Variant v, bool ta = false, bool tb = false);
+// solo: the launch has no more workgroups than the device has CUs (the 16-bit 128x128 DMA tiles then
+// take their form with three stage buffers).
+const void* kernelFor(Variant v, bool ta = false, bool tb = false, bool solo = false);
 // The one-pass skinny kernels (Variant::kGemv, kBf16Gemv, kFp16Gemv) for m
 // rows of a (up to the variant's row limit) and a row-major (ta false) or,
 // fp32 only, column-major a; null otherwise.  `threads` receives the
@@ -295,8 +297,8 @@ const void* dma32KernelTB(Variant v);  // column-major b
 const void* dma32KernelTA(Variant v, bool tb);  // column-major a
 const void* dmaKernelBf16(bool ta, bool tb);
 const void* dmaKernelFp16(bool ta, bool tb);
-const void* dma128KernelBf16(bool ta, bool tb, bool split);
-const void* dma128KernelFp16(bool ta, bool tb, bool split);
+const void* dma128KernelBf16(bool ta, bool tb, bool split, bool solo);
+const void* dma128KernelFp16(bool ta, bool tb, bool split, bool solo);
 const void* dma64x128KernelBf16(bool ta, bool tb);  // null for a column-major a
 const void* dma64x128KernelFp16(bool ta, bool tb);
 const void* groupedDmaKernelBf16(bool ta, bool tb);
