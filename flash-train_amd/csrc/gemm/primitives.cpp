@@ -262,12 +262,12 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
                                     : p.d().numericType() == FTRAIN_NUMERIC_TYPE_BF16 ? gemm::kCdBf16
                                                                                      : gemm::kCdFp16;
             reduce_ = ReduceParams{nullptr, g.c, g.d, alpha, beta, count, s.n, g.ldc, g.ldd, int32_t(splits), cd_type};
-            // isApplicable guaranteed n, ldc, ldd % 4 == 0 and 16-byte bases
-            // for the fp32 vec variants; the half variants reduce four at a
-            // time when c and d are fp32 and meet the same conditions.
-            const auto a16 = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-            reduce_vec_ = info_->vec && (!half_ || (!cd_half && s.n % 4 == 0 && g.ldd % 4 == 0 && a16(g.d) &&
-                                                    (g.c == nullptr || (g.ldc % 4 == 0 && a16(g.c)))));
+            // isApplicable guaranteed n, ldc, ldd % 4 == 0 and 16-byte bases for the fp32 vec variants;
+            // the half variants reduce four at a time when c and d meet the same conditions (four
+            // 16-bit elements are 8 bytes).
+            const uintptr_t quad = cd_half ? 8 : 16;
+            reduce_vec_ = info_->vec && (!half_ || (s.n % 4 == 0 && g.ldd % 4 == 0 && aligned(g.d, quad) &&
+                                                    (g.c == nullptr || (g.ldc % 4 == 0 && aligned(g.c, quad)))));
             const uint64_t units = reduce_vec_ ? count / 4 : count;
             // One thread per unit also when there are few splits: the 16-thread form then idles
             // most of its threads (measured on MI355X, 65536 float4 units: 2.6 against 2.9 us at

@@ -1,0 +1,93 @@
+"""Every 16-bit Primitive at the edges of its tiles, stages and store widths.
+
+Integer inputs, so every product and partial sum is exact in fp32 (k * 16 < 2^24) and d must be the
+exact result bit for bit: for a 16-bit d, its rounding to nearest even.  Operands lie in storages
+padded with NaN, so a read past a row that feeds a result fails the comparison, and d in one filled
+with a marker, so a store outside the matrix does too.
+"""
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+DT = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
+MARK = 77.0
+
+
+@pytest.fixture(scope="module")
+def capi():
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a visible device")
+    from flash_train import capi as c
+
+    return c
+
+
+@pytest.fixture(scope="module")
+def ops(capi):
+    return capi.GemmOps()
+
+
+def store(rows, cols, col_major, dtype, pad, shift, fill):
+    """A rows x cols view, row- or column-major, `shift` elements into a storage with `pad` spare
+    elements per leading dimension."""
+    r, c = (cols, rows) if col_major else (rows, cols)
+    whole = torch.full((r * (c + pad) + shift,), fill, dtype=dtype, device="cuda")
+    view = whole[shift:].view(r, c + pad)[:, :c]
+    return (view.t() if col_major else view), whole
+
+
+def check(capi, ops, kind, cd, m, n, k, ta, tb, with_c, ab_pad=0, ab_shift=0, cd_pad=0, cd_shift=0, only=None):
+    dtype, out = DT[kind], DT[cd]
+    gen = torch.Generator(device="cuda").manual_seed(m * 7 + n * 5 + k)
+
+    def ints(rows, cols):
+        return torch.randint(-4, 5, (rows, cols), generator=gen, device="cuda")
+
+    ai, bi, ci = ints(m, k), ints(k, n), ints(m, n)
+    a, _ = store(m, k, ta, dtype, ab_pad, ab_shift, float("nan"))
+    b, _ = store(k, n, tb, dtype, ab_pad, ab_shift, float("nan"))
+    c, _ = store(m, n, False, out, cd_pad, cd_shift, float("nan"))
+    d, whole = store(m, n, False, out, cd_pad, cd_shift, MARK)
+    a.copy_(ai), b.copy_(bi), c.copy_(ci)
+    want = 0.5 * (ai.double() @ bi.double()) + (2.0 * ci.double() if with_c else 0.0)
+    want = want.float().to(out)
+    outside = torch.ones_like(whole, dtype=torch.bool)
+    outside[cd_shift:].view(m, n + cd_pad)[:, :n] = False
+    plan = capi.plan_for(a, b, c if with_c else None, d, 0.5, 2.0, ops)
+    names = plan.names()
+    for i, name in enumerate(names):
+        if only is not None and only not in name:
+            continue
+        d.fill_(float("nan"))
+        plan.execute(i, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        where = f"{name} {kind} {cd} {m}x{n}x{k} ta={ta} tb={tb} c={with_c} pads {ab_pad} {ab_shift} {cd_pad} {cd_shift}"
+        assert torch.equal(d, want), f"{where}: {int((d != want).sum())} wrong"
+        assert bool((whole[outside] == MARK).all()), f"{where}: stored outside d"
+    return names
+
+
+# One, two, three and more stages of 64 k with and without a tail; one tile, a tile less and more a
+# row, several tiles; c and d in 16-byte units, and not (odd leading dimension, unaligned base).
+@pytest.mark.parametrize("kind,cd", [("bf16", "bf16"), ("bf16", "fp32"), ("fp16", "fp16")])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_half_tile_edges(capi, ops, kind, cd, ta, tb):
+    for m, n, k in ((256, 256, 64), (248, 264, 128), (264, 248, 136), (512, 520, 328), (8, 520, 40), (136, 136, 704)):
+        for with_c, pad, shift in ((False, 0, 0), (True, 0, 0), (True, 8, 8), (True, 3, 1), (False, 4, 4)):
+            check(capi, ops, kind, cd, m, n, k, ta, tb, with_c, cd_pad=pad, cd_shift=shift)
+    if not ta:  # rows free
+        check(capi, ops, kind, cd, 255, 264, 200, ta, tb, True)
+        check(capi, ops, kind, cd, 1, 264, 72, ta, tb, True)
+    if tb:  # columns free
+        check(capi, ops, kind, cd, 256, 255, 200, ta, tb, True)
+        check(capi, ops, kind, cd, 264, 130, 1032, ta, tb, True)
+
+
+# Launches of at most one workgroup per CU (three stage buffers) and of more, 1 to 7 stages, whole-k.
+@pytest.mark.parametrize("m,n", [(128, 128), (2048, 2048), (2048, 2176)])
+def test_half_128_tile_stage_counts(capi, ops, m, n):
+    for k in (40, 64, 128, 192, 200, 256, 320, 384, 456):
+        check(capi, ops, "bf16", "fp32", m, n, k, False, True, False, only="128x128_Dma")
