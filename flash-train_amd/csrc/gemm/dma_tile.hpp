@@ -208,7 +208,8 @@ static __device__ __attribute__((aligned(256))) u16 dma_dummy[512];
 // to slice z of p.d (dense m x n); the reduction kernel forms d.
 // BM: tile rows (T by default; 64 with T = 128 for m of at most 64, row-major a only).
 // NB: stage buffers; a stage's DMAs run NB - 1 stages ahead of its use.
-template <bool BF16, bool TA, bool TB, int T = 128, bool SPLIT = false, int BM = T, int NB = 2>
+// ROTATE: neighbouring column tiles start at different stages (the kernel below says why).
+template <bool BF16, bool TA, bool TB, int T = 128, bool SPLIT = false, int BM = T, int NB = 2, bool ROTATE = false>
 // band: tile rows per band of the tile order (tile_of).
 __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int bid, int z = 0, int band = 8) {
     constexpr bool A_TR = TA, B_TR = !TB;
@@ -279,8 +280,11 @@ __device__ __forceinline__ void half_gemm_dma_tile(const HalfGemmParams& p, int 
     constexpr int NRA = (A_TR ? 4 : 2) * NBM, NRB = (B_TR ? 4 : 2) * NBN, NR = NRA + NRB;
     constexpr int NM = 2 * NBM * NBN;  // MFMAs per half stage
     constexpr int ND = NDA + NDB;      // DMAs per wave per stage
-    // DMA d (0 .. ND - 1) of a stage: A and B alternate while both have some left.
+    // ROTATE: the workgroup walks its stages from stage `first` on and wraps around.
+    const int first = ROTATE && nst > 0 ? (3 * tn) % nst : 0;
+    // DMA d (0 .. ND - 1) of the st-th stage walked: A and B alternate while both have some left.
     auto dma_one = [&](int st, int d, int buf) {
+        if constexpr (ROTATE) st = st + first < nst ? st + first : max(st + first - nst, 0);
         constexpr int PAIRS = NDA < NDB ? NDA : NDB;
         const unsigned da = la + buf * kStageA * 2, db = lb + buf * kStageB * 2;
         if (d < 2 * PAIRS) {
@@ -496,6 +500,13 @@ __global__ __launch_bounds__(256, SOLO ? 1 : 2) void half_gemm_dma128(HalfGemmPa
 // splits: 6.7 us for the GEMM kernel against 8.0 us on the 128x128 split tile.  Three stage
 // buffers (72 KiB, still two workgroups per CU), each stage's DMAs issued two stages ahead:
 // 12.2 / 11.6 us per step with row- / column-major b against 12.8 / 12.3 with two.
+// Column-major b: every workgroup reads 128 columns, one line of each per stage, and with the columns
+// a power of two apart in memory all workgroups at the same stage meet in the same few HBM channels.
+// Neighbouring column tiles therefore start three stages apart and wrap around (the sum's order
+// changes with the tile, not from run to run): GEMM kernel alone, weights from HBM, 16x14336x4096 at 2
+// splits 27.1 -> 21.5 us (5.4 TB/s), 32x8192x8192 at 4 splits 34.6 -> 27.3; 64x4096x4096, whose b
+// comes from the last-level cache, unchanged (8.2).  A row-major b's stage is 256-byte runs of
+// consecutive rows and does not meet this (12.4 against 12.5 at 2 splits).
 template <bool BF16, bool TB>
 __global__ __launch_bounds__(256, 2) void half_gemm_dma64x128(HalfGemmParams p) {
     int bid = blockIdx.x, z = blockIdx.z;
@@ -507,7 +518,7 @@ __global__ __launch_bounds__(256, 2) void half_gemm_dma64x128(HalfGemmParams p) 
         const int t   = w - z * tiles, per = tiles >> 3;
         bid           = t < (per << 3) ? ((t % per) << 3) + t / per : t;
     }
-    half_gemm_dma_tile<BF16, false, TB, 128, true, 64, 3>(p, bid, z);
+    half_gemm_dma_tile<BF16, false, TB, 128, true, 64, 3, TB>(p, bid, z);
 }
 
 // Grouped GEMM over a device table of per-group parameters: the workgroup's

@@ -314,13 +314,14 @@ __global__ __launch_bounds__(256) void splitk_reduce(ReduceParams p) {
 
 // The same reduction with one thread per output unit, summing the slices in
 // increasing z: for outputs with enough units to fill the chip on their own
-// (the 16-thread form leaves 15 of 16 threads idle at two splits).
+// (the 16-thread form leaves 15 of 16 threads idle at two splits).  Blocks of
+// 256 threads, or of 64 for few units (wideReduceBlock).
 template <bool VEC>
 __global__ __launch_bounds__(256) void splitk_reduce_wide(ReduceParams p) {
     using V               = std::conditional_t<VEC, floatx4, float>;
     const uint64_t units  = VEC ? p.count / 4 : p.count;
     const V* __restrict__ W = reinterpret_cast<const V*>(p.partials);
-    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < units; i += (uint64_t)gridDim.x * 256) {
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < units; i += (uint64_t)gridDim.x * blockDim.x) {
         // Up to 8 slices' loads in flight before their adds (in increasing z): the pass is
         // latency-bound, a load per add kept one or two in flight.
         V s = W[i];

@@ -273,9 +273,10 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
             // most of its threads (measured on MI355X, 65536 float4 units: 2.6 against 2.9 us at
             // 4 splits, 3.3 at 8).
             reduce_wide_         = units >= gemm::kWideReduceUnits || splits <= 8;
-            // splitk_reduce: 16 output units per block (16 threads each); the
-            // wide form 256 units per block.
-            aux_grid_ = dim3(static_cast<uint32_t>(std::min<uint64_t>(ceilDiv(units, reduce_wide_ ? 256 : 16), 65535)));
+            // splitk_reduce: 16 output units per block (16 threads each); the wide form one unit per
+            // thread.
+            aux_block_ = dim3(reduce_wide_ ? gemm::wideReduceBlock(units) : 256);
+            aux_grid_  = dim3(static_cast<uint32_t>(std::min<uint64_t>(ceilDiv(units, reduce_wide_ ? aux_block_.x : 16), 65535)));
         }
     }
 
@@ -316,7 +317,7 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
                 void* rargs[]      = {&red};
                 hipError_t e       = hipLaunchKernel(kernel_, grid_, block_, args, 0, r.stream);
                 if (e == hipSuccess)
-                    e = hipLaunchKernel(gemm::reduceKernel(reduce_vec_, reduce_wide_), aux_grid_, dim3(256), rargs, 0, r.stream);
+                    e = hipLaunchKernel(gemm::reduceKernel(reduce_vec_, reduce_wide_), aux_grid_, aux_block_, rargs, 0, r.stream);
                 check(e, info_->name);
                 break;
             }
@@ -369,7 +370,7 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
     bool half_;  // bf16 / fp16 inputs (HalfGemmParams)
     bool empty_         = true;
     const void* kernel_ = nullptr;
-    dim3 grid_, block_, aux_grid_;
+    dim3 grid_, block_, aux_grid_, aux_block_;
     GemmParams params_{};
     HalfGemmParams half_params_{};
     WideParams wide_{};

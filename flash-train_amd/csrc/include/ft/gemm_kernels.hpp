@@ -329,6 +329,9 @@ const void* groupedHalfKernelFp16TT(int which);
 // per unit.
 const void* reduceKernel(bool vec, bool wide);
 constexpr uint64_t kWideReduceUnits = 256 * 1024;
+// Threads per block of the wide form: 64 while blocks of 256 would leave CUs without one (16384 units,
+// 16x4096 from 8 slices, are 64 such blocks).
+constexpr uint32_t wideReduceBlock(uint64_t units) { return units < 256 * 256 ? 64 : 256; }
 const void* deepkKernel();              // kDeepK64x64 (DeepKParams)
 const void* deepkClearKernel();         // zeroes (unsigned*, int n) arrival counters
 
