@@ -37,6 +37,12 @@ constexpr VariantInfo kInfo[] = {
     {"Fp32Mfma16Gemm_64x64_Dma_SplitK", 64, 64, 32, 256, 5, true, P, false, false, false, 0.964, FP32, 256.0, 0.846},
     {"Fp32Mfma16Gemm_64x128_Dma", 64, 128, 32, 256, 3, true, N, false, false, false, 0.966, FP32, 256.0, 0.933},
     {"Fp32Mfma16Gemm_128x64_Dma", 128, 64, 32, 256, 3, true, N, false, false, false, 0.933, FP32, 256.0, 0.934},
+    {"Fp32Mfma16Gemm_128x128_Dma_Unaligned", 128, 128, 32, 256, 2, false, N, false, false, false, 0.96, FP32, 256.0, 0.93},
+    {"Fp32Mfma16Gemm_128x128_Dma_Unaligned_SplitK", 128, 128, 32, 256, 2, false, P, false, false, false, 0.97, FP32, 256.0, 0.95},
+    {"Fp32Mfma16Gemm_64x128_Dma_Unaligned", 64, 128, 32, 256, 3, false, N, false, false, false, 0.94, FP32, 256.0, 0.91},
+    {"Fp32Mfma16Gemm_64x128_Dma_Unaligned_SplitK", 64, 128, 32, 256, 3, false, P, false, false, false, 0.94, FP32, 256.0, 0.87},
+    {"Fp32Mfma16Gemm_128x64_Dma_Unaligned_SplitK", 128, 64, 32, 256, 3, false, P, false, false, false, 0.92, FP32, 256.0, 0.93},
+    {"Fp32Mfma16Gemm_64x64_Dma_Unaligned_SplitK", 64, 64, 32, 256, 5, false, P, false, false, false, 0.94, FP32, 256.0, 0.82},
     {"Fp32Mfma16Gemm_256x256", 256, 256, 16, 256, 1, true, N, false, false, true, 0.903, FP32, 256.0, 0.903},
     {"Fp32Mfma16Gemm_256x256_SplitK", 256, 256, 16, 256, 1, true, P, false, false, true, 0.842, FP32, 256.0, 0.842},
     {"Fp32Mfma16Gemm_256x128", 256, 128, 16, 256, 2, true, N, false, false, true, 0.891, FP32, 256.0, 0.821},
@@ -75,10 +81,10 @@ constexpr VariantInfo kInfo[] = {
     {"Fp16MfmaGemm_64x64_Unaligned", 64, 64, 32, 256, 2, false, N, false, false, true, 0.08, FP16, 4096.0, 0.08},
     {"Bf16MfmaGemm_256x256_Dma", 256, 256, 64, 512, 1, true, N, false, false, true, 0.66, BF16, 4096.0, 0.66},
     {"Fp16MfmaGemm_256x256_Dma", 256, 256, 64, 512, 1, true, N, false, false, true, 0.66, FP16, 4096.0, 0.66},
-    {"Bf16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, BF16, 4096.0, 0.65},
-    {"Bf16MfmaGemm_128x128_Dma_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.55, BF16, 4096.0, 0.65},
-    {"Fp16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, FP16, 4096.0, 0.65},
-    {"Fp16MfmaGemm_128x128_Dma_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.55, FP16, 4096.0, 0.65},
+    {"Bf16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, BF16, 4096.0, 0.60},
+    {"Bf16MfmaGemm_128x128_Dma_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.55, BF16, 4096.0, 0.50},
+    {"Fp16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, FP16, 4096.0, 0.60},
+    {"Fp16MfmaGemm_128x128_Dma_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.55, FP16, 4096.0, 0.50},
     // Applicable to m of at most 64 only.  The low single-workgroup figure makes the model spread
     // such a problem over 8 splits (one workgroup per CU), as measured (64x4096x4096: 4 splits
     // leave half the CUs idle).
@@ -92,5 +98,7 @@ static_assert(sizeof(kInfo) / sizeof(kInfo[0]) == static_cast<int>(Variant::kCou
 }  // namespace
 
 const VariantInfo& info(Variant v) { return kInfo[static_cast<int>(v)]; }
+
+bool unsplitForm(Variant v) { return v == Variant::kMfma16Dma64x64S || v == Variant::kMfma16Dma64x64US; }
 
 }  // namespace ftrain::gemm

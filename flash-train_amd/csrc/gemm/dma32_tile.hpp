@@ -118,12 +118,19 @@ constexpr int kPartialPolicy = 2;
 // leading dimensions taken as 0, every lane's offset stays within 1 KiB of it.
 static __device__ __attribute__((aligned(256))) float dma32_dummy[512];
 
-template <int BM, int BN, int WM, int WN, bool SPLIT, bool TB = false, bool TA = false>
+// U: rows need no 16-byte alignment and n no multiple of 4 (row-major a only).  A multi-dword access
+// needs its address aligned to a dword only, so the DMAs and the epilogue keep their 16 bytes; what
+// changes is the 16-byte chunks that cross an edge of the matrix.  A chunk of b's columns that would
+// (n not a multiple of 4) is read from the row's last 4 columns instead, and the epilogue of a last
+// column tile, element by element, puts its values where they belong; a k tail's crossing chunks are
+// staged element by element.
+template <int BM, int BN, int WM, int WN, bool SPLIT, bool TB = false, bool TA = false, bool U = false>
 __device__ __forceinline__ void fp32_gemm_dma_tile(const GemmParams& p, int bid, int z, int band = 4) {
     static_assert(WM * WN == 4, "4 waves");
     constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16, NC = TN / 4;
     static_assert(TN % 4 == 0 && TM >= 1, "column runs of four blocks");
     static_assert(!TA || TM % 4 == 0, "row runs of four blocks");
+    static_assert(!U || !TA, "unaligned tiles take row-major a");
     constexpr int RA = 256 / BM;       // k rows per A DMA (column-major a)
     constexpr int CPA = BM / 4;        // 16-byte chunks per A k row (column-major a)
     constexpr bool ASWZ = CPA >= 32;
@@ -171,13 +178,15 @@ __device__ __forceinline__ void fp32_gemm_dma_tile(const GemmParams& p, int bid,
     const char* abase_r   = reinterpret_cast<const char*>(p.a + (size_t)m0 * lda_r + kbeg);
     const char* abase     = none ? dummy : abase_r;
     // B block q = wave + 4 j: k rows RB q .. RB q + RB - 1 (lane: row RB q + lane / CPR), slot
-    // lane % CPR holds chunk (lane % CPR) ^ swizzle; a chunk past n is clamped onto the last whole
-    // one (n % 4 == 0).  x = the swizzle bit of the block's k rows.
-    const char* bbase_r = reinterpret_cast<const char*>(p.b + (size_t)kbeg * ldb_r + n0);
+    // lane % CPR holds chunk (lane % CPR) ^ swizzle; a chunk past n, or across it, is clamped onto the
+    // last 4 columns (n >= 4; nb is the leftmost column read).  x = the swizzle bit of the block's k
+    // rows.
+    const int nb        = U ? min(n0, N - 4) : n0;
+    const char* bbase_r = reinterpret_cast<const char*>(p.b + (size_t)kbeg * ldb_r + nb);
     const char* bbase   = none ? dummy : bbase_r;
     auto boff = [&](int x, int64_t ld) {
         const int kr = lane / CPR, chunk = (lane % CPR) ^ (x ? 16 : 0);
-        return static_cast<unsigned>((kr * ld + (min(n0 + 4 * chunk, N - 4) - n0)) * 4);
+        return static_cast<unsigned>((kr * ld + (min(n0 + 4 * chunk, N - 4) - nb)) * 4);
     };
     const unsigned boff0 = boff(0, ldb), boff1 = BSWZ ? boff(1, ldb) : boff0;
     // Column-major a: block q = wave + 4 j holds k rows RA q .. RA q + RA - 1 of the stage (lane: k
@@ -377,9 +386,19 @@ __device__ __forceinline__ void fp32_gemm_dma_tile(const GemmParams& p, int bid,
         // like a whole stage.
         if (k_tail > 0) {
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            auto put = [&](float* stage, int q, bool ok, const char* src) {
+            // left: how many of the chunk's elements lie before kend (only a k-contiguous chunk of an
+            // unaligned tile can hold some of both kinds).
+            typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+            auto put = [&](float* stage, int q, int left, const char* src) {
                 floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
-                if (ok) v = *reinterpret_cast<const floatx4*>(src);
+                if (left >= 4) {
+                    v = U ? *reinterpret_cast<const floatx4u*>(src) : *reinterpret_cast<const floatx4*>(src);
+                } else if (U && left > 0) {
+                    const float* e = reinterpret_cast<const float*>(src);
+                    v[0]           = e[0];
+                    if (left > 1) v[1] = e[1];
+                    if (left > 2) v[2] = e[2];
+                }
                 *reinterpret_cast<floatx4*>(reinterpret_cast<char*>(stage) + q * 1024 + 16 * lane) = v;
             };
             const size_t st_k = (size_t)nst * kStageK;
@@ -389,10 +408,10 @@ __device__ __forceinline__ void fp32_gemm_dma_tile(const GemmParams& p, int bid,
                 if constexpr (TA) {
                     const int kr0 = RA * q;
                     const unsigned off = aoff(ASWZ && ((kr0 >> 3) & 1), lda_r);
-                    put(As0, q, kr0 + lane / CPA < k_tail, atbase_r + (st_k + kr0) * lda_r * 4 + off);
+                    put(As0, q, kr0 + lane / CPA < k_tail ? 4 : 0, atbase_r + (st_k + kr0) * lda_r * 4 + off);
                 } else {
                     const unsigned row = min(ar + 32u * j, alast);
-                    put(As0, q, int(achunk / 4) < k_tail,
+                    put(As0, q, k_tail - int(achunk / 4),
                         abase_r + st_k * 4 + (size_t)row * lda_r * 4 + achunk);
                 }
             }
@@ -404,11 +423,11 @@ __device__ __forceinline__ void fp32_gemm_dma_tile(const GemmParams& p, int bid,
                     const int cb = 4 * ((lane >> 3) & 1) + 2 * (lane >> 5) + (t & 1);
                     const int ch = 4 * (t >> 2) + 2 * ((lane >> 4) & 1) + ((t >> 1) & 1);
                     const unsigned col = min(static_cast<unsigned>(8 * q + cb), blast);
-                    put(Bs0, q, 4 * ch < k_tail, btbase_r + st_k * 4 + (size_t)col * ldb_r * 4 + 16 * ch);
+                    put(Bs0, q, k_tail - 4 * ch, btbase_r + st_k * 4 + (size_t)col * ldb_r * 4 + 16 * ch);
                 } else {
                     const int kr0 = RB * q;
                     const unsigned off = boff(BSWZ && ((kr0 >> 3) & 1), ldb_r);
-                    put(Bs0, q, kr0 + lane / CPR < k_tail, bbase_r + (st_k + kr0) * ldb_r * 4 + off);
+                    put(Bs0, q, kr0 + lane / CPR < k_tail ? 4 : 0, bbase_r + (st_k + kr0) * ldb_r * 4 + off);
                 }
             }
             __syncthreads();
@@ -443,12 +462,22 @@ __device__ __forceinline__ void fp32_gemm_dma_tile(const GemmParams& p, int bid,
     const unsigned lane_d = (GROW * g * ldd + 4 * j16) * 4, lane_c = (GROW * g * ldc + 4 * j16) * 4;
     // Row of lane group 0 for block row bi, register r.
     auto row_of = [&](int bi, int r) { return TA ? wrow + (bi >> 2) * 64 + 4 * r + (bi & 3) : wrow + 16 * bi + r; };
-    auto run = [&](auto c_tag) {
-        constexpr bool HAS_C = decltype(c_tag)::value;
+    // EDGE (unaligned tiles with columns past the matrix): element by element.  A chunk across the
+    // last column holds the 4 columns before the edge, `back` columns further left than its place;
+    // those of them that the chunk to its left has too are not stored again.
+    auto run = [&](auto c_tag, auto edge_tag) {
+        constexpr bool HAS_C = decltype(c_tag)::value, EDGE = decltype(edge_tag)::value;
         __amdgpu_buffer_rsrc_t cres = dres;
         if constexpr (HAS_C)
             cres = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.c) + (size_t)m0 * p.ldc + n0, 0,
                                                      span(p.ldc), kBufferConfig);
+        // EDGE: byte offset of element t of this lane's chunk at column c0 + 4 j16 (kOut if not stored).
+        auto edge_off = [&](int row0, int c0, int t, unsigned ld) {
+            const int col   = c0 + 4 * j16;
+            const int back  = !TB && col + 4 > cols_left ? col + 4 - cols_left : 0;
+            const bool mine = TB ? col + t < cols_left : col < cols_left && t >= back;
+            return GROW * g < rows_left - row0 && mine ? (GROW * g * ld + static_cast<unsigned>(col - back + t)) * 4 : kOut;
+        };
         floatx4 cv[HAS_C ? 2 : 1][4][NC];
         auto load_c = [&](int bi, floatx4 (&dst)[4][NC]) {
 #pragma unroll
@@ -456,11 +485,19 @@ __device__ __forceinline__ void fp32_gemm_dma_tile(const GemmParams& p, int bid,
                 const int row0 = row_of(bi, r);
 #pragma unroll
                 for (int q = 0; q < NC; ++q) {
-                    const int c0  = wcol + 64 * q;
-                    const bool ok = GROW * g < rows_left - row0 && c0 + 4 * j16 < cols_left;
-                    dst[r][q]     = __builtin_bit_cast(
-                        floatx4, __builtin_amdgcn_raw_buffer_load_b128(cres, ok ? lane_c : kOut,
-                                                                       static_cast<int>((row0 * ldc + c0) * 4), 0));
+                    const int c0 = wcol + 64 * q;
+                    if constexpr (EDGE) {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            dst[r][q][t] = __builtin_bit_cast(
+                                float, __builtin_amdgcn_raw_buffer_load_b32(cres, edge_off(row0, c0, t, ldc),
+                                                                            static_cast<int>(row0 * ldc * 4), 0));
+                    } else {
+                        const bool ok = GROW * g < rows_left - row0 && c0 + 4 * j16 < cols_left;
+                        dst[r][q]     = __builtin_bit_cast(
+                            floatx4, __builtin_amdgcn_raw_buffer_load_b128(cres, ok ? lane_c : kOut,
+                                                                           static_cast<int>((row0 * ldc + c0) * 4), 0));
+                    }
                 }
             }
         };
@@ -474,8 +511,7 @@ __device__ __forceinline__ void fp32_gemm_dma_tile(const GemmParams& p, int bid,
                 const int row0 = row_of(bi, r);
 #pragma unroll
                 for (int q = 0; q < NC; ++q) {
-                    const int c0  = wcol + 64 * q;
-                    const bool ok = GROW * g < rows_left - row0 && c0 + 4 * j16 < cols_left;
+                    const int c0 = wcol + 64 * q;
                     floatx4 out;
 #pragma unroll
                     for (int t = 0; t < 4; ++t) {
@@ -486,19 +522,40 @@ __device__ __forceinline__ void fp32_gemm_dma_tile(const GemmParams& p, int bid,
                             if constexpr (HAS_C) out[t] += beta * cv[HAS_C ? bi & 1 : 0][r][q][t];
                         }
                     }
-                    store_b128<SPLIT ? kPartialPolicy : 0>(out, dres, ok ? lane_d : kOut,
-                                                           static_cast<int>((row0 * ldd + c0) * 4));
+                    if constexpr (EDGE) {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            const float v = out[t];
+                            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), dres,
+                                                                  edge_off(row0, c0, t, ldd),
+                                                                  static_cast<int>(row0 * ldd * 4),
+                                                                  SPLIT ? kPartialPolicy : 0);
+                        }
+                    } else {
+                        const bool ok = GROW * g < rows_left - row0 && c0 + 4 * j16 < cols_left;
+                        store_b128<SPLIT ? kPartialPolicy : 0>(out, dres, ok ? lane_d : kOut,
+                                                               static_cast<int>((row0 * ldd + c0) * 4));
+                    }
                 }
             }
         }
     };
-    if (!SPLIT && p.c != nullptr)
-        run(std::true_type{});
-    else
-        run(std::false_type{});
+    auto run_edge = [&](auto edge_tag) {
+        if (!SPLIT && p.c != nullptr)
+            run(std::true_type{}, edge_tag);
+        else
+            run(std::false_type{}, edge_tag);
+    };
+    if constexpr (U) {
+        if (cols_left < BN) {
+            run_edge(std::true_type{});
+            return;
+        }
+    }
+    run_edge(std::false_type{});
 }
 
-template <int BM, int BN, int WM, int WN, int MINB, bool SPLIT, bool TB = false, bool TA = false>
+template <int BM, int BN, int WM, int WN, int MINB, bool SPLIT, bool TB = false, bool TA = false, bool U = false>
 __global__ __launch_bounds__(256, MINB) void fp32_gemm_dma(GemmParams p) {
     int bid = blockIdx.x, z = blockIdx.z;
     if constexpr (SPLIT) {
@@ -513,7 +570,7 @@ __global__ __launch_bounds__(256, MINB) void fp32_gemm_dma(GemmParams p) {
             bid           = t < (per << 3) ? ((t % per) << 3) + t / per : t;
         }
     }
-    fp32_gemm_dma_tile<BM, BN, WM, WN, SPLIT, TB, TA>(p, bid, z);
+    fp32_gemm_dma_tile<BM, BN, WM, WN, SPLIT, TB, TA, U>(p, bid, z);
 }
 
 // Grouped GEMM over a device table of per-group parameters (whole-k tiles): the workgroup's

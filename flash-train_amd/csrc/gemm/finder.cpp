@@ -60,8 +60,9 @@ constexpr double kCuBytesPerMicro = 6.4e4;  // one CU's sustained load rate (abo
 // pipeline has drained: per tile, the drain, the loads' latency and a barrier.  Fitted to the bf16
 // grouped weight gradient (16384 ragged tokens, 4096x14336 weights, ms, DMA against register-staged
 // 256x256 tile): 8 experts 1.80 / 2.01, 16 2.25 / 2.42, 32 3.28 / 3.23, 64 5.28 / 4.86, 128 9.15 /
-// 8.22; the DMA tile is ranked first at 8 experts only (7% lost at 16).
-constexpr double kDmaTailMicros = 3.0;
+// 8.22; the DMA tile is ranked first at 8 experts only (7% lost at 16).  A smaller tile stages as
+// much less: fp32 127x97x33 (one stage and a tail) takes 4.4 us in all on the 64x64 tile.
+constexpr double kDmaTailMicros = 3.0;  // of a 256x256 tile
 constexpr uint64_t kMinSplitDepth = 256;  // reduction depth worth one split-k workgroup
 constexpr uint64_t kMinGemvDepth  = 64;
 
@@ -109,7 +110,7 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
     double bytes      = eb * (m * k + k * n + m * n * (has_c ? 2.0 : 1.0));
     double launch     = kLaunchMicros;
     double serial_us  = 0.0;  // work in a second kernel that cannot overlap the first
-    if (vi.split == SplitKind::kPartial) {
+    if (vi.split == SplitKind::kPartial && (splits > 1 || vi.gemv)) {
         // The GEMM kernel writes splits partial tiles instead of d; the
         // reduction kernel then reads them (and c) and writes d.
         bytes += 4.0 * m * n * (double(splits) - 1.0 - (has_c ? 1.0 : 0.0));
@@ -163,7 +164,7 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
     const double tails     = !dmaTail(vi, s.k) ? 0.0 : used == 1 ? rounds
                                                    : double(ceilDiv(ceilDiv(tiles, cus), uint64_t(vi.occupancy)));
     const double compute   = double(per_cu) * 2.0 * vi.bm * vi.bn * depth / cu_rate + rounds * per_round +
-                           tails * kDmaTailMicros;
+                           tails * kDmaTailMicros * std::min(1.0, vi.bm * vi.bn / 65536.0);
     // A launch with fewer workgroups than CUs streams memory through only that many of them (a CU
     // moves a bounded number of bytes per clock): 64x4096x14336 bf16 on the 64x128 split tile took
     // 36.3 us at 4 splits (128 workgroups) against 23.8 us at 8.  On the 16-bit 64x128 split tile
@@ -179,7 +180,8 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
     // tile (32 workgroups of 0.5 MiB) 9.3 us against 13.2 for the split tile the fraction picked,
     // 128x256x512 6.5 against 10.7 for the 64x64 unaligned tile.  At 224 workgroups (4x28672x4096)
     // the fraction still ranks right.
-    if (vi.split == SplitKind::kNone && !vi.simt && 2 * wgs <= uint64_t(cus)) {
+    if ((vi.split == SplitKind::kNone || (vi.split == SplitKind::kPartial && splits == 1)) && !vi.simt &&
+        2 * wgs <= uint64_t(cus)) {
         const double wg_bytes = eb * double(vi.bm + vi.bn) * double(s.k) + 4.0 * vi.bm * vi.bn;
         memory = std::max(bytes / kHbmBytesPerMicro, wg_bytes / kCuBytesPerMicro);
     }
@@ -232,16 +234,22 @@ uint32_t chooseSplits(Variant v, const GemmShape& s, int cus) {
         return static_cast<uint32_t>(best);
     }
     if (vi.gemv && most < 2) return 1;  // the skinny kernel also runs unsplit
-    if (most < 2 || s.m == 0 || s.n == 0) return 0;
-    // Smallest modelled time over powers of two in [2, most] (ties: fewer splits).
+    if (s.m == 0 || s.n == 0) return 0;
+    // Smallest modelled time over 2^i and 3 * 2^i in [2, most] (ties: fewer splits), and 1 for a tile
+    // with a whole-k form.
     uint64_t best = 0;
     double best_t = std::numeric_limits<double>::infinity();
-    for (uint64_t sp = 2; sp <= most; sp *= 2) {
+    const auto consider = [&](uint64_t sp) {
         const double t = modelMicros(vi, s, false, cus, sp);
         if (t < best_t * 0.999) {
             best_t = t;
             best   = sp;
         }
+    };
+    if (unsplitForm(v)) consider(1);
+    for (uint64_t sp = 2; sp <= most; sp *= 2) {
+        consider(sp);
+        if (!vi.gemv && sp + sp / 2 <= most) consider(sp + sp / 2);
     }
     return static_cast<uint32_t>(best);
 }

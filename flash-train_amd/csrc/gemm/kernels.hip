@@ -419,7 +419,8 @@ const void* gemvKernel(Variant v, int m, bool ta, int& threads) {
     return ta ? reinterpret_cast<const void*>(&gemv_pass<8, 2, 8, true>) : reinterpret_cast<const void*>(&gemv_pass<8, 2, 8, false>);
 }
 
-const void* kernelFor(Variant v, bool ta, bool tb, bool solo) {
+const void* kernelFor(Variant v, bool ta, bool tb, bool solo, bool whole) {
+    if (whole) return ta ? nullptr : v == Variant::kMfma16Dma64x64S ? dma32Kernel64x64(tb) : dma32Kernel64x64U(tb);
     if (info(v).gemv && info(v).split == SplitKind::kNone) {
         if (tb) return nullptr;
         int threads = 0;
@@ -440,6 +441,7 @@ const void* kernelFor(Variant v, bool ta, bool tb, bool solo) {
         return table[i / kHalfTiles][(ta ? 1 : 0) + (tb ? 2 : 0)](tile);
     }
     if (v >= Variant::kMfma16Dma256x256 && v <= Variant::kMfma16Dma128x64) return ta ? dma32KernelTA(v, tb) : tb ? dma32KernelTB(v) : dma32Kernel(v);
+    if (v >= Variant::kMfma16Dma128x128U && v <= Variant::kMfma16Dma64x64US) return ta ? nullptr : dma32KernelU(v, tb);
     if (v == Variant::kBf16MfmaDma256x256) return dmaKernelBf16(ta, tb);
     if (v == Variant::kFp16MfmaDma256x256) return dmaKernelFp16(ta, tb);
     if (v == Variant::kBf16MfmaDma128x128 || v == Variant::kBf16MfmaDma128x128S)

@@ -20,6 +20,11 @@ const void* dma32Kernel(Variant v) {
     }
 }
 
+const void* dma32Kernel64x64(bool tb) {
+    return tb ? reinterpret_cast<const void*>(&d32::fp32_gemm_dma<64, 64, 4, 1, 2, false, true>)
+              : reinterpret_cast<const void*>(&d32::fp32_gemm_dma<64, 64, 4, 1, 2, false>);
+}
+
 const void* groupedDma32Kernel() {
     return reinterpret_cast<const void*>(&d32::grouped_fp32_gemm_dma<256, 256, 2, 2, 1, false, false>);
 }

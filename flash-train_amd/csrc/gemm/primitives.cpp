@@ -77,6 +77,18 @@ Result commonChecks(const GemmProblem& p, FTrainNumericType input) {
     return Result{};
 }
 
+// Whether every fp32 matrix takes 128-bit accesses along its contiguous dimension: that extent and
+// the leading dimension a multiple of 4, the base 16-byte aligned.
+bool fits128(const GemmProblem& p, const GemmLaunch& g) {
+    const GemmShape s    = g.shape;
+    const uint64_t a_run = g.ta ? s.m : s.k, b_run = g.tb ? s.k : s.n;
+    if (s.n % 4 != 0 || a_run % 4 != 0 || b_run % 4 != 0) return false;
+    if (g.lda % 4 != 0 || g.ldb % 4 != 0 || g.ldc % 4 != 0 || g.ldd % 4 != 0) return false;
+    for (int i = 0; i < 4; ++i)
+        if (!vecAligned(p.port(i).memory())) return false;
+    return true;
+}
+
 // The launch's workgroup size must equal the kernel's launch bounds (every
 // kernel here declares its exact size: a larger launch fails, a smaller one
 // would leave part of each tile uncomputed).  Checked when HIP can describe
@@ -165,7 +177,12 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
                 if (!vecAligned(p.port(i).memory()))
                     return Result(FTRAIN_STATUS_UNSUPPORTED, "a matrix address is not 16-byte aligned");
         }
-        if (v_ >= Variant::kMfma16Dma256x256 && v_ <= Variant::kMfma16Dma128x64 &&
+        if (v_ >= Variant::kMfma16Dma128x128U && v_ <= Variant::kMfma16Dma64x64US) {
+            if (s.n < 4) return Result(FTRAIN_STATUS_UNSUPPORTED, "n below 4 (16-byte loads of a row of b)");
+            if (fits128(p, g))
+                return Result(FTRAIN_STATUS_UNSUPPORTED, "every operand fits 128-bit accesses (the aligned DMA tiles take it)");
+        }
+        if (v_ >= Variant::kMfma16Dma256x256 && v_ <= Variant::kMfma16Dma64x64US &&
             (s.k == 0 || g.lda >= (int64_t(1) << 22) || g.ldb >= (int64_t(1) << 22) || g.ldc >= (int64_t(1) << 21) ||
              g.ldd >= (int64_t(1) << 21)))
             return Result(FTRAIN_STATUS_UNSUPPORTED,
@@ -243,7 +260,8 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
             params_.tiles_m = half_params_.tiles_m = int32_t(ceilDiv(s.m, info_->bm));
             params_.tiles_n = half_params_.tiles_n = int32_t(ceilDiv(s.n, info_->bn));
             grid_           = dim3(uint32_t(params_.tiles_m) * uint32_t(params_.tiles_n), 1, splits);
-            kernel_         = gemm::kernelFor(v_, g.ta, g.tb, uint64_t(grid_.x) * splits <= uint64_t(cus));
+            unsplit_        = splits == 1 && gemm::unsplitForm(v_);
+            kernel_         = gemm::kernelFor(v_, g.ta, g.tb, uint64_t(grid_.x) * splits <= uint64_t(cus), unsplit_);
         }
         const uint64_t count = s.m * s.n;
         if (info_->split == SplitKind::kFused) {
@@ -256,18 +274,17 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
             partial_bytes_ = splits > 1 ? gemm::kCounterBytes + uint64_t(splits) * tiles * info_->bm * info_->bn * sizeof(float) : 0;
             fused_tiles_   = int32_t(tiles);
         }
-        if (info_->split == SplitKind::kPartial) {
+        if (info_->split == SplitKind::kPartial && !unsplit_) {
             partial_bytes_ = gemm::kCounterBytes + uint64_t(splits) * count * sizeof(float);
             const int32_t cd_type = !cd_half ? gemm::kCdFp32
                                     : p.d().numericType() == FTRAIN_NUMERIC_TYPE_BF16 ? gemm::kCdBf16
                                                                                      : gemm::kCdFp16;
             reduce_ = ReduceParams{nullptr, g.c, g.d, alpha, beta, count, s.n, g.ldc, g.ldd, int32_t(splits), cd_type};
-            // isApplicable guaranteed n, ldc, ldd % 4 == 0 and 16-byte bases for the fp32 vec variants;
-            // the half variants reduce four at a time when c and d meet the same conditions (four
-            // 16-bit elements are 8 bytes).
+            // The reduction takes four elements at a time where c and d allow (four 16-bit elements
+            // are 8 bytes).
             const uintptr_t quad = cd_half ? 8 : 16;
-            reduce_vec_ = info_->vec && (!half_ || (s.n % 4 == 0 && g.ldd % 4 == 0 && aligned(g.d, quad) &&
-                                                    (g.c == nullptr || (g.ldc % 4 == 0 && aligned(g.c, quad)))));
+            reduce_vec_ = s.n % 4 == 0 && g.ldd % 4 == 0 && aligned(g.d, quad) &&
+                          (g.c == nullptr || (g.ldc % 4 == 0 && aligned(g.c, quad)));
             const uint64_t units = reduce_vec_ ? count / 4 : count;
             // One thread per unit also when there are few splits: the 16-thread form then idles
             // most of its threads (measured on MI355X, 65536 float4 units: 2.6 against 2.9 us at
@@ -291,7 +308,7 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
         GemmParams params          = params_;
         HalfGemmParams half_params = half_params_;
         void* args[]               = {half_ ? static_cast<void*>(&half_params) : static_cast<void*>(&params)};
-        switch (info_->split) {
+        switch (unsplit_ ? SplitKind::kNone : info_->split) {
             case SplitKind::kNone:
                 check(hipLaunchKernel(kernel_, grid_, block_, args, 0, r.stream), info_->name);
                 break;
@@ -377,6 +394,7 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
     ReduceParams reduce_{};
     gemm::DeepKParams deepk_{};
     int32_t fused_tiles_ = 0;
+    bool unsplit_           = false;  // a split-k variant in its whole-k form (gemm::unsplitForm)
     bool reduce_vec_        = false;
     bool reduce_wide_       = false;
     uint64_t partial_bytes_ = 0;

@@ -138,6 +138,14 @@ enum class Variant : int {
     kMfma16Dma64x64S,
     kMfma16Dma64x128,
     kMfma16Dma128x64,
+    // The same for operands without 16-byte alignment (any n of at least 4,
+    // row-major a): whole-k and split-k.
+    kMfma16Dma128x128U,
+    kMfma16Dma128x128US,
+    kMfma16Dma64x128U,
+    kMfma16Dma64x128US,
+    kMfma16Dma128x64US,
+    kMfma16Dma64x64US,
     kMfma16_256x256,
     kMfma16_256x256S,
     // Same instruction, 256x128 tiles of 4 waves of 128x64, two workgroups
@@ -260,7 +268,11 @@ const VariantInfo& info(Variant v);
 // instantiated for the variant (see VariantInfo::layouts).
 // solo: the launch has no more workgroups than the device has CUs (the 16-bit 128x128 DMA tiles then
 // take their form with three stage buffers).
-const void* kernelFor(Variant v, bool ta = false, bool tb = false, bool solo = false);
+// whole: the whole-k form of a split-k variant that may run unsplit (unsplitForm).
+const void* kernelFor(Variant v, bool ta = false, bool tb = false, bool solo = false, bool whole = false);
+// Whether a split-k variant may also run with one split: it then launches its whole-k form, which
+// writes d itself (no workspace, no reduction).  The fp32 64x64 DMA tiles, aligned and not.
+bool unsplitForm(Variant v);
 // The one-pass skinny kernels (Variant::kGemv, kBf16Gemv, kFp16Gemv) for m
 // rows of a (up to the variant's row limit) and a row-major (ta false) or,
 // fp32 only, column-major a; null otherwise.  `threads` receives the
@@ -290,11 +302,14 @@ const void* halfKernelFp16NT(int tile);
 const void* halfKernelFp16TT(int tile);
 // The DMA-staged 256x256 tiles per input type and operand orientation.
 const void* dma32Kernel(Variant v);
+const void* dma32Kernel64x64(bool tb);  // the whole-k form of kMfma16Dma64x64S
 const void* groupedDma32Kernel();
 const void* groupedDma32Kernel128(bool ta, bool tb);  // grouped 128x128 DMA tile, any orientation
 const void* groupedDma32Kernel64x128(bool tb);        // grouped 64x128 DMA tile, row-major a
 const void* dma32KernelTB(Variant v);  // column-major b
 const void* dma32KernelTA(Variant v, bool tb);  // column-major a
+const void* dma32KernelU(Variant v, bool tb);   // unaligned operands, row-major a
+const void* dma32Kernel64x64U(bool tb);         // the whole-k form of kMfma16Dma64x64US
 const void* dmaKernelBf16(bool ta, bool tb);
 const void* dmaKernelFp16(bool ta, bool tb);
 const void* dma128KernelBf16(bool ta, bool tb, bool split, bool solo);

@@ -91,3 +91,31 @@ def test_half_tile_edges(capi, ops, kind, cd, ta, tb):
 def test_half_128_tile_stage_counts(capi, ops, m, n):
     for k in (40, 64, 128, 192, 200, 256, 320, 384, 456):
         check(capi, ops, "bf16", "fp32", m, n, k, False, True, False, only="128x128_Dma")
+
+
+# fp32 without 16-byte alignment: rows, columns and depths of every remainder by 4, one to several
+# stages of 32 k, tile edges crossed by 1, 2 and 3 columns, unaligned bases and leading dimensions.
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("m,n,k", [(127, 97, 33), (128, 129, 31), (65, 130, 1), (129, 131, 64), (64, 4, 101), (3, 5, 7),
+                                   (200, 255, 130), (257, 385, 1027), (64, 128, 2050)])
+def test_fp32_unaligned_tiles(capi, ops, tb, m, n, k):
+    for with_c, ab_pad, ab_shift, cd_pad, cd_shift in ((False, 0, 0, 0, 0), (True, 0, 0, 0, 0), (True, 1, 1, 3, 2),
+                                                       (True, 4, 1, 0, 1), (False, 2, 3, 5, 3)):
+        names = check(capi, ops, "fp32", "fp32", m, n, k, False, tb, with_c, ab_pad, ab_shift, cd_pad, cd_shift)
+        assert "Fp32Mfma16Gemm_128x128_Dma_Unaligned" in names, names
+
+
+def test_fp32_unaligned_in_place(capi, ops):
+    # c and d one matrix, a last column tile of 1, 2 and 3 columns: every element read before it is written once.
+    for n in (129, 130, 131):
+        a = torch.randint(-4, 5, (200, 70), device="cuda").float()
+        b = torch.randint(-4, 5, (70, n), device="cuda").float()
+        c = torch.randint(-4, 5, (200, n), device="cuda").float()
+        want = (0.5 * (a.double() @ b.double()) + 2.0 * c.double()).float()
+        d = c.clone()
+        plan = capi.plan_for(a, b, d, d, 0.5, 2.0, ops)
+        for i, name in enumerate(plan.names()):
+            d.copy_(c)
+            plan.execute(i, torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            assert torch.equal(d, want), (name, n)
