@@ -105,7 +105,12 @@ __device__ __forceinline__ void tile_of(int bid, int tiles_m, int tiles_n, int& 
 // z of the workspace (dense m x n) for splitk_reduce.
 // ----------------------------------------------------------------------------
 // The tile body (see mfma_tile.hpp): tile `bid` of p's grid, split `z`.
-template <bool BF16, int BM, int BN, int BK, int WM, int WN, int MINB, bool VEC, int SPLIT, bool TA, bool TB>
+// U (with VEC): 16-byte loads at any 2-byte aligned address (gfx950 takes unaligned global loads),
+// for rows that are not multiples of 8 elements.  A chunk of 8 columns of a row-major b (rows of a
+// column-major a) must not cross the matrix edge, so the last tile is moved left (up) until it ends
+// with the matrix, which needs n (m) of at least a tile; the outputs it shares with its neighbour are
+// not stored.  A k tail's crossing chunks are the last 8 elements of their rows, shifted.
+template <bool BF16, int BM, int BN, int BK, int WM, int WN, int MINB, bool VEC, int SPLIT, bool TA, bool TB, bool U = false>
 __device__ __forceinline__ void half_gemm_tile(const HalfGemmParams& p, int bid, int z) {
     using u16           = unsigned short;
     constexpr int NT    = WM * WN * 64;
@@ -151,8 +156,10 @@ __device__ __forceinline__ void half_gemm_tile(const HalfGemmParams& p, int bid,
 
     int tm, tn;
     tile_of(bid, p.tiles_m, p.tiles_n, tm, tn);
-    const int m0 = tm * BM, n0 = tn * BN;
     const int M = p.m, N = p.n, K = p.k;
+    // First row and column of the tile, and the first ones it stores.
+    const int mt = tm * BM, nt = tn * BN;
+    const int m0 = U && TA ? min(mt, M - BM) : mt, n0 = U && !TB ? min(nt, N - BN) : nt;
     const int kbeg = SPLIT != kWhole ? z * p.k_chunk : 0;
     const int kend = SPLIT != kWhole ? min(K, kbeg + p.k_chunk) : K;
     const int nst  = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
@@ -187,6 +194,21 @@ __device__ __forceinline__ void half_gemm_tile(const HalfGemmParams& p, int bid,
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
     const u32x4 zero4 = u32x4{0u, 0u, 0u, 0u};
+    typedef u32x4 u32x4_any __attribute__((aligned(2)));
+    // 16 bytes of a row; `left` elements of them lie before kend (8 or more unless a k tail's chunk).
+    auto load16 = [&](const u16* src, int left) {
+        if constexpr (!U) return *reinterpret_cast<const u32x4*>(src);
+        // A crossing chunk: the row's last 8 elements before kend (k is at least a stage), shifted down
+        // so that zeros follow the ones that belong to the chunk.
+        const int over  = left < 8 ? 8 - left : 0;
+        const u32x4 v   = *reinterpret_cast<const u32x4_any*>(src - over);
+        const uint64_t lo = v[0] | static_cast<uint64_t>(v[1]) << 32, hi = v[2] | static_cast<uint64_t>(v[3]) << 32;
+        const int sh    = 16 * over;
+        const uint64_t l = sh == 0 ? lo : sh < 64 ? lo >> sh | hi << (64 - sh) : hi >> (sh - 64);
+        const uint64_t h = sh < 64 ? hi >> sh : 0;
+        return u32x4{static_cast<unsigned>(l), static_cast<unsigned>(l >> 32), static_cast<unsigned>(h),
+                     static_cast<unsigned>(h >> 32)};
+    };
 
     // Stages [k_lo, k_lo + n_st * BK), the last one cut at kend.
     auto main_loop = [&](auto checked_tag, const int k_lo, const int n_st) {
@@ -212,12 +234,12 @@ __device__ __forceinline__ void half_gemm_tile(const HalfGemmParams& p, int bid,
                         const int r = idx / (BK / 8), kq = 8 * (idx % (BK / 8));
                         const int gm = row_at(m0 + r, M, 1), gk = k0 + kq;
                         ra[j][0] = zero4;
-                        if (!CHECKED || (gm < M && gk < kend)) ra[j][0] = *reinterpret_cast<const u32x4*>(a_at(gm, gk));
+                        if (!CHECKED || (gm < M && gk < kend)) ra[j][0] = load16(a_at(gm, gk), CHECKED ? kend - gk : 8);
                     } else {  // (k, 8 m) vectors along the contiguous m
                         const int k = idx / (BM / 8), mq = 8 * (idx % (BM / 8));
                         const int gm = row_at(m0 + mq, M, 8), gk = k0 + k;
                         ra[j][0] = zero4;
-                        if (!CHECKED || (gm < M && gk < kend)) ra[j][0] = *reinterpret_cast<const u32x4*>(a_at(gm, gk));
+                        if (!CHECKED || (gm < M && gk < kend)) ra[j][0] = load16(a_at(gm, gk), 8);
                     }
                 }
 #pragma unroll
@@ -229,12 +251,12 @@ __device__ __forceinline__ void half_gemm_tile(const HalfGemmParams& p, int bid,
                         const int c = idx / (BK / 8), kq = 8 * (idx % (BK / 8));
                         const int gn = row_at(n0 + c, N, 1), gk = k0 + kq;
                         rb[j][0] = zero4;
-                        if (!CHECKED || (gn < N && gk < kend)) rb[j][0] = *reinterpret_cast<const u32x4*>(b_at(gk, gn));
+                        if (!CHECKED || (gn < N && gk < kend)) rb[j][0] = load16(b_at(gk, gn), CHECKED ? kend - gk : 8);
                     } else {  // (k, 8 n) vectors along the contiguous n
                         const int k = idx / (BN / 8), nq = 8 * (idx % (BN / 8));
                         const int gn = row_at(n0 + nq, N, 8), gk = k0 + k;
                         rb[j][0] = zero4;
-                        if (!CHECKED || (gn < N && gk < kend)) rb[j][0] = *reinterpret_cast<const u32x4*>(b_at(gk, gn));
+                        if (!CHECKED || (gn < N && gk < kend)) rb[j][0] = load16(b_at(gk, gn), 8);
                     }
                 }
             } else {
@@ -483,7 +505,7 @@ __device__ __forceinline__ void half_gemm_tile(const HalfGemmParams& p, int bid,
                     for (int r = 0; r < 16; ++r) {
                         const int row     = m0 + wrow + bi * 32 + 8 * (r / 4) + 4 * h + (r % 4);
                         const size_t ci   = (size_t)row * p.ldc + col;
-                        const bool inside = col < N && row < M;
+                        const bool inside = col < N && row < M && (!U || (col >= nt && row >= mt));
                         if constexpr (HALF)
                             dst[t][r] = inside ? to_float<BF16>(static_cast<const u16*>(p.c)[ci]) : 0.f;
                         else
@@ -501,11 +523,11 @@ __device__ __forceinline__ void half_gemm_tile(const HalfGemmParams& p, int bid,
 #pragma unroll
                 for (int t = 0; t < UB; ++t) {
                     const int col = n0 + wcol + (bj0 + t) * 32 + li;
-                    if (col >= N) continue;
+                    if (col >= N || (U && col < nt)) continue;
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const int row = m0 + wrow + bi * 32 + 8 * (r / 4) + 4 * h + (r % 4);
-                        if (row >= M) continue;
+                        if (row >= M || (U && row < mt)) continue;
                         const size_t di = (size_t)row * p.ldd + col;
                         float out       = alpha * acc[bi][bj0 + t][r];
                         if constexpr (HAS_C) out += beta * cv[HAS_C ? u & 1 : 0][t][r];
@@ -535,9 +557,9 @@ __device__ __forceinline__ void half_gemm_tile(const HalfGemmParams& p, int bid,
     }
 }
 
-template <bool BF16, int BM, int BN, int BK, int WM, int WN, int MINB, bool VEC, int SPLIT, bool TA, bool TB>
+template <bool BF16, int BM, int BN, int BK, int WM, int WN, int MINB, bool VEC, int SPLIT, bool TA, bool TB, bool U = false>
 __global__ __launch_bounds__(WM* WN * 64, MINB) void half_gemm(HalfGemmParams p) {
-    half_gemm_tile<BF16, BM, BN, BK, WM, WN, MINB, VEC, SPLIT, TA, TB>(p, blockIdx.x, blockIdx.z);
+    half_gemm_tile<BF16, BM, BN, BK, WM, WN, MINB, VEC, SPLIT, TA, TB, U>(p, blockIdx.x, blockIdx.z);
 }
 
 // Grouped GEMM over a device table of per-group parameters (see
@@ -596,6 +618,9 @@ const void* halfKernel(int tile) {
         case 2:
             return reinterpret_cast<const void*>(&half_gemm<BF16, 128, 128, 64, 2, 2, 2, true, kPartial, TA, TB>);
         case 3: return reinterpret_cast<const void*>(&half_gemm<BF16, 64, 64, 32, 2, 2, 2, false, kWhole, TA, TB>);
+        // The large tile of the _Unaligned variant (kHalfUnaligned128).
+        case kHalfUnaligned128:
+            return reinterpret_cast<const void*>(&half_gemm<BF16, 128, 128, 64, 2, 2, 2, true, kWhole, TA, TB, true>);
         default: return nullptr;
     }
 }

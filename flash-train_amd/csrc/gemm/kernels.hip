@@ -419,6 +419,14 @@ const void* gemvKernel(Variant v, int m, bool ta, int& threads) {
     return ta ? reinterpret_cast<const void*>(&gemv_pass<8, 2, 8, true>) : reinterpret_cast<const void*>(&gemv_pass<8, 2, 8, false>);
 }
 
+const void* halfUnaligned128(bool bf16, bool ta, bool tb) {
+    if (bf16)
+        return ta ? (tb ? halfKernelBf16TT(kHalfUnaligned128) : halfKernelBf16TN(kHalfUnaligned128))
+                  : (tb ? halfKernelBf16NT(kHalfUnaligned128) : halfKernelBf16NN(kHalfUnaligned128));
+    return ta ? (tb ? halfKernelFp16TT(kHalfUnaligned128) : halfKernelFp16TN(kHalfUnaligned128))
+              : (tb ? halfKernelFp16NT(kHalfUnaligned128) : halfKernelFp16NN(kHalfUnaligned128));
+}
+
 const void* kernelFor(Variant v, bool ta, bool tb, bool solo, bool whole) {
     if (whole) return ta ? nullptr : v == Variant::kMfma16Dma64x64S ? dma32Kernel64x64(tb) : dma32Kernel64x64U(tb);
     if (info(v).gemv && info(v).split == SplitKind::kNone) {

@@ -89,6 +89,18 @@ bool fits128(const GemmProblem& p, const GemmLaunch& g) {
     return true;
 }
 
+// Whether the 16-bit per-element variant runs a problem on its 128x128 tile (16-byte loads at any
+// address).  A row-major b needs n, a column-major a m of at least a tile (the kernel moves its last
+// tile inside the matrix).  The large tile costs more before its first and after its last stage, so a
+// short k needs many tiles: bf16, us, per-element tile against it: 1000x5003x2048 87 / 41,
+// 1533x14043x3340 (both column-major, 16-bit c) 862 / 296, 526x1575x630 20.7 / 14.4, 300x1001x1000
+// 27.9 / 16.8, but 200x201x200 8.8 / 9.8 and 150x301x70 5.8 / 9.0.
+bool takes128(const GemmLaunch& g) {
+    const GemmShape s = g.shape;
+    if (s.m <= 64 || s.n <= 64 || (g.ta && s.m < 128) || (!g.tb && s.n < 128)) return false;
+    return s.k >= 256 || (s.k >= 128 && ceilDiv(s.m, 64) * ceilDiv(s.n, 64) > 512);
+}
+
 // The launch's workgroup size must equal the kernel's launch bounds (every
 // kernel here declares its exact size: a larger launch fails, a smaller one
 // would leave part of each tile uncomputed).  Checked when HIP can describe
@@ -260,6 +272,14 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
             params_.tiles_m = half_params_.tiles_m = int32_t(ceilDiv(s.m, info_->bm));
             params_.tiles_n = half_params_.tiles_n = int32_t(ceilDiv(s.n, info_->bn));
             grid_           = dim3(uint32_t(params_.tiles_m) * uint32_t(params_.tiles_n), 1, splits);
+            const bool per_element = v_ == Variant::kBf16Mfma64x64U || v_ == Variant::kFp16Mfma64x64U;
+            if (per_element && takes128(g)) {
+                half_params_.tiles_m = int32_t(ceilDiv(s.m, 128));
+                half_params_.tiles_n = int32_t(ceilDiv(s.n, 128));
+                grid_   = dim3(uint32_t(half_params_.tiles_m) * uint32_t(half_params_.tiles_n));
+                kernel_ = gemm::halfUnaligned128(v_ == Variant::kBf16Mfma64x64U, g.ta, g.tb);
+                return;
+            }
             unsplit_        = splits == 1 && gemm::unsplitForm(v_);
             kernel_         = gemm::kernelFor(v_, g.ta, g.tb, uint64_t(grid_.x) * splits <= uint64_t(cus), unsplit_);
         }

@@ -226,6 +226,9 @@ enum class Variant : int {
 // order of the four variants above): 0 = 256x256, 1 = 128x128,
 // 2 = 128x128 split-k, 3 = 64x64 per-element.
 constexpr int kHalfTiles = 4;
+// Index of the 128x128 tile that the 64x64 per-element variant runs on when the problem is large
+// enough for it (16-byte loads at unaligned addresses).
+constexpr int kHalfUnaligned128 = 4;
 
 enum class SplitKind : int {
     kNone,     // one workgroup owns each output tile's whole reduction
@@ -270,6 +273,8 @@ const VariantInfo& info(Variant v);
 // take their form with three stage buffers).
 // whole: the whole-k form of a split-k variant that may run unsplit (unsplitForm).
 const void* kernelFor(Variant v, bool ta = false, bool tb = false, bool solo = false, bool whole = false);
+// The 16-bit per-element variants' 128x128 tile (kHalfUnaligned128).
+const void* halfUnaligned128(bool bf16, bool ta, bool tb);
 // Whether a split-k variant may also run with one split: it then launches its whole-k form, which
 // writes d itself (no workspace, no reduction).  The fp32 64x64 DMA tiles, aligned and not.
 bool unsplitForm(Variant v);

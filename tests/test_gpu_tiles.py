@@ -119,3 +119,32 @@ def test_fp32_unaligned_in_place(capi, ops):
             plan.execute(i, torch.cuda.current_stream().cuda_stream)
             torch.cuda.synchronize()
             assert torch.equal(d, want), (name, n)
+
+
+# 16-bit rows that are not multiples of 8 elements: problems on the per-element 64x64 tile and, from
+# 128 rows or columns of a transposed operand on, on its 128x128 form, whose last tile moves inside the
+# matrix; k tails of 1 to 63, unaligned bases and leading dimensions.
+@pytest.mark.parametrize("kind,cd", [("bf16", "fp32"), ("fp16", "fp16")])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_half_unaligned_tiles(capi, ops, kind, cd, ta, tb):
+    for m, n, k in ((129, 131, 257), (128, 128, 259), (255, 257, 319), (300, 129, 383), (131, 300, 320), (65, 66, 100),
+                    (127, 127, 300), (66, 500, 333), (1500, 1601, 129)):
+        for with_c, ab_pad, ab_shift, cd_pad in ((True, 0, 0, 0), (False, 3, 1, 1), (True, 1, 5, 3)):
+            names = check(capi, ops, kind, cd, m, n, k, ta, tb, with_c, ab_pad, ab_shift, cd_pad, 1 if cd_pad else 0,
+                          only="Unaligned")
+            assert any("64x64_Unaligned" in nm for nm in names), names
+
+
+def test_half_unaligned_in_place(capi, ops):
+    # c and d one matrix: the outputs that a moved last tile shares with its neighbour are written once.
+    a = torch.randint(-4, 5, (300, 301), device="cuda").bfloat16()
+    b = torch.randint(-4, 5, (301, 301), device="cuda").bfloat16()
+    c = torch.randint(-4, 5, (300, 301), device="cuda").float()
+    want = (0.5 * (a.double() @ b.double()) + 2.0 * c.double()).float()
+    d = c.clone()
+    plan = capi.plan_for(a, b, d, d, 0.5, 2.0, ops)
+    for i, name in enumerate(plan.names()):
+        d.copy_(c)
+        plan.execute(i, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(d, want), name
