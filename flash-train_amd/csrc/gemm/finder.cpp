@@ -63,10 +63,20 @@ constexpr double kCuBytesPerMicro = 6.4e4;  // one CU's sustained load rate (abo
 // 8.22; the DMA tile is ranked first at 8 experts only (7% lost at 16).  A smaller tile stages as
 // much less: fp32 127x97x33 (one stage and a tail) takes 4.4 us in all on the 64x64 tile.
 constexpr double kDmaTailMicros = 3.0;  // of a 256x256 tile
+// Rate of a lone workgroup of the 16-bit 128x128 DMA tiles in their form for two per CU.
+constexpr double kPairedSoloEfficiency = 0.37;
 constexpr uint64_t kMinSplitDepth = 256;  // reduction depth worth one split-k workgroup
 constexpr uint64_t kMinGemvDepth  = 64;
 
 uint64_t ceilDiv(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
+
+// Rows of a problem in tile rows of vi.  The 16-bit 256x256 DMA tile runs a last tile row of at most
+// 128 rows at half the cost.
+double tileRows(const VariantInfo& vi, uint64_t m) {
+    const uint64_t rows = ceilDiv(m, vi.bm), left = m - (rows ? rows - 1 : 0) * vi.bm;
+    const bool halves   = vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 256 && std::strstr(vi.name, "_Dma") != nullptr;
+    return halves && left <= 128 ? double(rows) - 0.5 : double(rows);
+}
 
 // Whether variant vi runs a k tail through the separate pass of the DMA tiles (stages of 32 k for
 // fp32, 64 for 16-bit inputs).
@@ -163,8 +173,16 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
     // The tail pass: every tile's when whole-k, the last split's tiles when split.
     const double tails     = !dmaTail(vi, s.k) ? 0.0 : used == 1 ? rounds
                                                    : double(ceilDiv(ceilDiv(tiles, cus), uint64_t(vi.occupancy)));
-    const double compute   = double(per_cu) * 2.0 * vi.bm * vi.bn * depth / cu_rate + rounds * per_round +
-                           tails * kDmaTailMicros * std::min(1.0, vi.bm * vi.bn / 65536.0);
+    double mfma = double(per_cu) * 2.0 * vi.bm * vi.bn * depth / cu_rate;
+    // The 16-bit 128x128 DMA tiles between one and two workgroups per CU: a second workgroup costs a
+    // CU half of what the first does, and only some CUs hold one (bf16, k 4096: 288 tiles 45 us, 384 52,
+    // 512 60).
+    if (vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 128 && std::strstr(vi.name, "_Dma") != nullptr &&
+        wgs > uint64_t(cus) && wgs <= 2 * uint64_t(cus)) {
+        const double one = mfma / 2.0 * residentEfficiency(vi, 2) / kPairedSoloEfficiency;
+        mfma             = one + (mfma - one) * (double(wgs) / double(cus) - 1.0);
+    }
+    const double compute   = mfma + rounds * per_round + tails * kDmaTailMicros * std::min(1.0, vi.bm * vi.bn / 65536.0);
     // A launch with fewer workgroups than CUs streams memory through only that many of them (a CU
     // moves a bounded number of bytes per clock): 64x4096x14336 bf16 on the 64x128 split tile took
     // 36.3 us at 4 splits (128 workgroups) against 23.8 us at 8.  On the 16-bit 64x128 split tile
@@ -273,7 +291,7 @@ double groupedMicros(Variant v, const std::vector<GemmShape>& shapes, bool has_c
         const uint64_t t = ceilDiv(s.m, vi.bm) * ceilDiv(s.n, vi.bn);
         tiles += t;
         if (dmaTail(vi, s.k)) tail_tiles += t;
-        flops += double(t) * 2.0 * vi.bm * vi.bn * double(std::max<uint64_t>(s.k, vi.bk));
+        flops += tileRows(vi, s.m) * double(ceilDiv(s.n, vi.bn)) * 2.0 * vi.bm * vi.bn * double(std::max<uint64_t>(s.k, vi.bk));
         bytes += eb * (double(s.m) * s.k + double(s.k) * s.n + double(s.m) * s.n * (has_c ? 2.0 : 1.0));
     }
     if (tiles == 0) return kLaunchMicros;
