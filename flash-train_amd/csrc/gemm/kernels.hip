@@ -209,6 +209,83 @@ __global__ __launch_bounds__(NW * 64) void gemv_pass(GemmParams p) {
 }
 
 // ----------------------------------------------------------------------------
+// One-pass skinny-m kernel for a column-major b (m <= MR <= 8, row-major a; k,
+// lda, ldb multiples of 4, 16-byte aligned a and b): the x @ w^T of a linear
+// layer's weight.  A wave takes 4 columns of b over all of k; a step is 256 k
+// of each, 1 KiB contiguous per load, U steps loaded before any is used, with
+// the same k of every row of a.  Each lane sums its own k and a butterfly over
+// the wave finishes the 4 x m sums, which go straight to d.  Neighbouring
+// waves start at different steps and wrap around: at one step, columns a power
+// of two apart would meet in the same HBM channels.
+// ----------------------------------------------------------------------------
+template <int U, int MR>
+__global__ __launch_bounds__(512) void gemv_pass_tb(GemmParams p) {
+    constexpr int C = 4;
+    static_assert(8 * C == kGemvPassCols, "columns per workgroup");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int M = p.m, N = p.n, K = p.k;
+    const int col0 = blockIdx.x * kGemvPassCols + wave * C;
+    if (col0 >= N) return;
+    // Columns past n and rows past m are read at a clamped index; they feed only sums that are not stored.
+    const float* b[C];
+    const float* a[MR];
+#pragma unroll
+    for (int c = 0; c < C; ++c) b[c] = p.b + (size_t)min(col0 + c, N - 1) * p.ldb + 4 * lane;
+#pragma unroll
+    for (int i = 0; i < MR; ++i) a[i] = p.a + (size_t)min(i, M - 1) * p.lda + 4 * lane;
+    float acc[MR][C];
+#pragma unroll
+    for (int i = 0; i < MR; ++i)
+#pragma unroll
+        for (int c = 0; c < C; ++c) acc[i][c] = 0.f;
+    auto load = [&](int k, floatx4 (&bv)[C], floatx4 (&av)[MR], bool in) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) bv[c] = in ? *reinterpret_cast<const floatx4*>(b[c] + k) : floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < MR; ++i) av[i] = in ? *reinterpret_cast<const floatx4*>(a[i] + k) : floatx4{0.f, 0.f, 0.f, 0.f};
+    };
+    auto fma = [&](const floatx4 (&bv)[C], const floatx4 (&av)[MR]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < MR; ++i)
+#pragma unroll
+                for (int c = 0; c < C; ++c) acc[i][c] += av[i][t] * bv[c][t];
+    };
+    // Whole groups of U steps, from group `first` on; then what is left of k.
+    const int groups = K / (256 * U);
+    int at           = groups > 0 ? (3 * (8 * blockIdx.x + wave)) % groups : 0;
+    for (int s = 0; s < groups; ++s) {
+        floatx4 bv[U][C], av[U][MR];
+#pragma unroll
+        for (int u = 0; u < U; ++u) load((at * U + u) * 256, bv[u], av[u], true);
+#pragma unroll
+        for (int u = 0; u < U; ++u) fma(bv[u], av[u]);
+        at = at + 1 < groups ? at + 1 : 0;
+    }
+    for (int k = groups * 256 * U; k < K; k += 256) {
+        floatx4 bv[C], av[MR];
+        load(k, bv, av, k + 4 * lane < K);
+        fma(bv, av);
+    }
+#pragma unroll
+    for (int sh = 1; sh < 64; sh <<= 1)
+#pragma unroll
+        for (int i = 0; i < MR; ++i)
+#pragma unroll
+            for (int c = 0; c < C; ++c) acc[i][c] += __shfl_xor(acc[i][c], sh);
+    // Every lane holds every sum: lane 4 i + c stores row i, column c.
+    float mine = 0.f;
+#pragma unroll
+    for (int i = 0; i < MR; ++i)
+#pragma unroll
+        for (int c = 0; c < C; ++c) mine = lane == C * i + c ? acc[i][c] : mine;
+    const int row = lane / C, col = col0 + lane % C;
+    if (row < M && row < MR && col < N)
+        p.d[(size_t)row * p.ldd + col] = p.alpha * mine + (p.c != nullptr ? p.beta * p.c[(size_t)row * p.ldc + col] : 0.f);
+}
+
+// ----------------------------------------------------------------------------
 // Split-k reduction: d = alpha * sum_{z < splits} W[z] + (c ? beta*c : 0) in a
 // fixed summation order (deterministic).  The slices are dense m x n fp32; c
 // and d are row-major with row strides ldc and ldd, in fp32 or a 16-bit type
@@ -410,9 +487,17 @@ __global__ __launch_bounds__(256) void simt_gemm(WideParams p) {
 // and 16 x 2, spill registers there).  The 16-bit kernel uses the same.
 int gemvPassThreads(int m) { return m <= 1 || m > 4 ? 512 : 1024; }
 
-const void* gemvKernel(Variant v, int m, bool ta, int& threads) {
+const void* gemvKernel(Variant v, int m, bool ta, bool tb, int& threads) {
     threads = gemvPassThreads(m);
-    if (v == Variant::kBf16Gemv || v == Variant::kFp16Gemv) return ta ? nullptr : gemvHalfKernel(v == Variant::kBf16Gemv, m);
+    if (v == Variant::kBf16Gemv || v == Variant::kFp16Gemv) return ta || tb ? nullptr : gemvHalfKernel(v == Variant::kBf16Gemv, m);
+    if (tb) {
+        threads = 512;
+        if (ta) return nullptr;
+        if (m <= 1) return reinterpret_cast<const void*>(&gemv_pass_tb<4, 1>);
+        if (m <= 2) return reinterpret_cast<const void*>(&gemv_pass_tb<4, 2>);
+        if (m <= 4) return reinterpret_cast<const void*>(&gemv_pass_tb<2, 4>);
+        return reinterpret_cast<const void*>(&gemv_pass_tb<2, 8>);
+    }
     if (m <= 1) return ta ? reinterpret_cast<const void*>(&gemv_pass<8, 2, 1, true>) : reinterpret_cast<const void*>(&gemv_pass<8, 2, 1, false>);
     if (m <= 2) return ta ? reinterpret_cast<const void*>(&gemv_pass<16, 2, 2, true>) : reinterpret_cast<const void*>(&gemv_pass<16, 2, 2, false>);
     if (m <= 4) return ta ? reinterpret_cast<const void*>(&gemv_pass<16, 2, 4, true>) : reinterpret_cast<const void*>(&gemv_pass<16, 2, 4, false>);
@@ -430,9 +515,8 @@ const void* halfUnaligned128(bool bf16, bool ta, bool tb) {
 const void* kernelFor(Variant v, bool ta, bool tb, bool solo, bool whole) {
     if (whole) return ta ? nullptr : v == Variant::kMfma16Dma64x64S ? dma32Kernel64x64(tb) : dma32Kernel64x64U(tb);
     if (info(v).gemv && info(v).split == SplitKind::kNone) {
-        if (tb) return nullptr;
         int threads = 0;
-        return gemvKernel(v, kGemvRows, ta, threads);
+        return gemvKernel(v, kGemvRows, ta, tb, threads);
     }
     if (v >= Variant::kMfma16_256x256 && v <= Variant::kMfma16_256x64S) {
         using Fn                     = const void* (*)(int);

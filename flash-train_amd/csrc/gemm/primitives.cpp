@@ -214,6 +214,13 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
             return Result(FTRAIN_STATUS_UNSUPPORTED, "m above 64 (the 64-row tile is for shapes one tile high)");
         if (info_->gemv && s.m > uint64_t(info_->bm))
             return Result(FTRAIN_STATUS_UNSUPPORTED, "m exceeds the skinny-kernel row limit");
+        // Column-major b: with more rows each CU also reads more of a, so from three rows on the kernel
+        // needs a workgroup per CU (32 columns each) or a short k.  us, against the best DMA split-k tile:
+        // one row 8192^2 44.7 / 73.2, 14336x4096 42.7 / 65.5, 2048^2 6.0 / 10.4; two rows 45.8 / 73.8, 45.8 /
+        // 65.8, 7.1 / 10.5; four rows 8192^2 49.1 / 74.5, 1024^2 6.1 / 9.6, but 4096x14336 75 / 62; eight rows
+        // 8192^2 58.7 / 74.9, but 4096x8192 51.9 / 42.2 (n x k).
+        if (v_ == Variant::kGemv && g.tb && s.m > 2 && s.n < 8192 && (s.m > 4 || s.k > 2048))
+            return Result(FTRAIN_STATUS_UNSUPPORTED, "too few columns of a column-major b for this many rows (skinny kernel)");
         if (info_->split == SplitKind::kPartial &&
             gemm::chooseSplits(v_, s, gemm::computeUnits(constraints.device())) == 0)
             return Result(FTRAIN_STATUS_UNSUPPORTED, "reduction depth too shallow to split");
@@ -241,7 +248,7 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
         wide_ = WideParams{a, b, c, d, alpha, beta, s.m, s.n, s.k, a_rs, a_cs, b_rs, b_cs, g.ldc, g.ldd};
 
         int threads = info_->threads;
-        kernel_     = info_->gemv && info_->split == SplitKind::kNone ? gemm::gemvKernel(v_, int(s.m), g.ta, threads)
+        kernel_     = info_->gemv && info_->split == SplitKind::kNone ? gemm::gemvKernel(v_, int(s.m), g.ta, g.tb, threads)
                                                                   : gemm::kernelFor(v_, g.ta, g.tb);
         checkBlockSize(kernel_, threads, info_->name);
         block_  = dim3(threads);

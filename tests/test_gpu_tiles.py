@@ -148,3 +148,14 @@ def test_half_unaligned_in_place(capi, ops):
         plan.execute(i, torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
         assert torch.equal(d, want), name
+
+
+# The one-pass skinny kernel with a column-major b: every row count, columns across a workgroup's 32 and
+# a wave's 4, depths with and without whole groups of its steps, padded strides.
+@pytest.mark.parametrize("m", range(1, 9))
+def test_fp32_gemv_column_major_b(capi, ops, m):
+    for n, k in ((32, 256), (36, 1024), (4, 4), (100, 516), (200, 2052), (64, 4096), (1000, 3076), (8196, 516),
+                 (8192, 2308)):
+        for with_c, ab_pad, cd_pad in ((False, 0, 0), (True, 4, 8)):
+            names = check(capi, ops, "fp32", "fp32", m, n, k, False, True, with_c, ab_pad, 0, cd_pad, 0, only="Fp32Gemv")
+            assert ("Fp32Gemv" in names) == (m <= 2 or n >= 8192 or (m <= 4 and k <= 2048)), names
