@@ -70,6 +70,11 @@ constexpr uint64_t kMinGemvDepth  = 64;
 
 uint64_t ceilDiv(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
+// The 16-bit 64x128 split tile (m of at most 64).
+bool half64x128(const VariantInfo& vi) {
+    return vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 64 && vi.bn == 128 && vi.split == SplitKind::kPartial;
+}
+
 // Rows of a problem in tile rows of vi.  The 16-bit 256x256 DMA tile runs a last tile row of at most
 // 128 rows at half the cost.
 double tileRows(const VariantInfo& vi, uint64_t m) {
@@ -189,9 +194,7 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
     // (m of at most 64) 85% of the CUs already stream at the full rate: 32x14336x4096 22.5 us at 2
     // splits (224 workgroups) against 24.1 at 4, and 5-10% the same way at 4 to 64 rows of n 13824
     // and 14336; the 128x128 split tile at such counts lost 4-15%, so it keeps the plain fraction.
-    const bool half_64x128 = vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 64 && vi.bn == 128 &&
-                             vi.split == SplitKind::kPartial;
-    const double fill = std::min(1.0, double(wgs) / (double(cus) * (half_64x128 ? 0.85 : 1.0)));
+    const double fill = std::min(1.0, double(wgs) / (double(cus) * (half64x128(vi) ? 0.85 : 1.0)));
     double memory     = bytes / (kHbmBytesPerMicro * fill);
     // A whole-k launch of at most half as many workgroups as CUs is bound by what each workgroup
     // loads at one CU's rate, not by a fraction of HBM: bf16 128x4096x1024 on the 128x128 DMA
@@ -267,7 +270,10 @@ uint32_t chooseSplits(Variant v, const GemmShape& s, int cus) {
     if (unsplitForm(v)) consider(1);
     for (uint64_t sp = 2; sp <= most; sp *= 2) {
         consider(sp);
-        if (!vi.gemv && sp + sp / 2 <= most) consider(sp + sp / 2);
+        // Not for the 16-bit 64x128 tile: it streams from memory, and workgroups just past a multiple of
+        // the CUs cost it more than the finer choice gives (bf16, column-major b, us at 2 / 3 / 4 splits:
+        // 16x11008x5120 28.6 / 33.1 / 29.8, 4x13824x5120 30.6 / 35.2 / 32.6; 2x6016x8992 at 4 / 6 25.0 / 32.0).
+        if (!vi.gemv && !half64x128(vi) && sp + sp / 2 <= most) consider(sp + sp / 2);
     }
     return static_cast<uint32_t>(best);
 }
@@ -291,7 +297,10 @@ double groupedMicros(Variant v, const std::vector<GemmShape>& shapes, bool has_c
         const uint64_t t = ceilDiv(s.m, vi.bm) * ceilDiv(s.n, vi.bn);
         tiles += t;
         if (dmaTail(vi, s.k)) tail_tiles += t;
-        flops += tileRows(vi, s.m) * double(ceilDiv(s.n, vi.bn)) * 2.0 * vi.bm * vi.bn * double(std::max<uint64_t>(s.k, vi.bk));
+        // A tile with a k tail gains less from a short last row (3143 tokens over 7 experts, 5984 columns,
+        // k 1040: 256x256 DMA tile 86 us, register-staged 78).
+        const double rows = dmaTail(vi, s.k) ? double(ceilDiv(s.m, vi.bm)) : tileRows(vi, s.m);
+        flops += rows * double(ceilDiv(s.n, vi.bn)) * 2.0 * vi.bm * vi.bn * double(std::max<uint64_t>(s.k, vi.bk));
         bytes += eb * (double(s.m) * s.k + double(s.k) * s.n + double(s.m) * s.n * (has_c ? 2.0 : 1.0));
     }
     if (tiles == 0) return kLaunchMicros;
