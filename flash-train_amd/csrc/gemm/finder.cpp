@@ -54,6 +54,10 @@ constexpr double kFusedStoreMicros    = 2.0;  // per round: a split workgroup's 
 // Fixed cost per round of resident workgroups (operand prologue, epilogue
 // stores, the ramp of the first stages); fitted with the catalog efficiencies.
 constexpr double kRoundMicros     = 3.35;
+constexpr double kThinRoundMicros = 7.0;  // a second round on few CUs, see modelMicros
+// The 16-bit 256x256 DMA tile's sustained fraction in a grouped launch, which reads every group's own
+// weight from memory (MLP forward over 8 experts 0.53 of peak, plain 0.58-0.62).
+constexpr double kGroupedHalf256Efficiency = 0.66;
 constexpr double kTieWeight       = 1e-3;
 constexpr double kCuBytesPerMicro = 6.4e4;  // one CU's sustained load rate (about 27 bytes per clock)
 // A DMA tile stages a partial last stage (k not a multiple of its stage) by ordinary loads once its
@@ -75,12 +79,15 @@ bool half64x128(const VariantInfo& vi) {
     return vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 64 && vi.bn == 128 && vi.split == SplitKind::kPartial;
 }
 
+bool half256Dma(const VariantInfo& vi) {
+    return vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 256 && std::strstr(vi.name, "_Dma") != nullptr;
+}
+
 // Rows of a problem in tile rows of vi.  The 16-bit 256x256 DMA tile runs a last tile row of at most
 // 128 rows at half the cost.
 double tileRows(const VariantInfo& vi, uint64_t m) {
     const uint64_t rows = ceilDiv(m, vi.bm), left = m - (rows ? rows - 1 : 0) * vi.bm;
-    const bool halves   = vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 256 && std::strstr(vi.name, "_Dma") != nullptr;
-    return halves && left <= 128 ? double(rows) - 0.5 : double(rows);
+    return half256Dma(vi) && left <= 128 ? double(rows) - 0.5 : double(rows);
 }
 
 // Whether variant vi runs a k tail through the separate pass of the DMA tiles (stages of 32 k for
@@ -187,6 +194,14 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
         const double one = mfma / 2.0 * residentEfficiency(vi, 2) / kPairedSoloEfficiency;
         mfma             = one + (mfma - one) * (double(wgs) / double(cus) - 1.0);
     }
+    // A second round of 16-bit 256x256 tiles on a fifth of the CUs or fewer has nothing beside its loads
+    // and stores (bf16, 256x256 against 128x128 DMA tile, us: 12714x1344x1216 62.7 / 56.8, 1824x9088x640
+    // 37.4 / 33.4, 7789x2176x128 27.7 / 19.2; from k 4160 on the 256x256 tile wins: 8960x2048x4160 160 /
+    // 165, 12614x1408x5056 199 / 212).  Not where n leaves rows of odd 64-byte pieces, which the smaller
+    // tiles touch twice: 2048x9432x64 22.7 / 41.5, 7424x2328x256 32.8 / 37.8, 3584x5112x768 44 / 59.
+    if (vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 256 && s.n % 32 == 0 && wgs > uint64_t(cus) &&
+        5 * wgs <= 6 * uint64_t(cus))
+        mfma += kThinRoundMicros;
     const double compute   = mfma + rounds * per_round + tails * kDmaTailMicros * std::min(1.0, vi.bm * vi.bn / 65536.0);
     // A launch with fewer workgroups than CUs streams memory through only that many of them (a CU
     // moves a bounded number of bytes per clock): 64x4096x14336 bf16 on the 64x128 split tile took
@@ -305,7 +320,8 @@ double groupedMicros(Variant v, const std::vector<GemmShape>& shapes, bool has_c
     }
     if (tiles == 0) return kLaunchMicros;
     const uint64_t per_cu = ceilDiv(tiles, cus);
-    const double cu_rate  = vi.flop_per_clk * kClockPerMicro * residentEfficiency(vi, per_cu);
+    const double cu_rate  = vi.flop_per_clk * kClockPerMicro *
+                            (half256Dma(vi) ? kGroupedHalf256Efficiency : residentEfficiency(vi, per_cu));
     const double rounds   = double(ceilDiv(per_cu, uint64_t(vi.occupancy)));
     const double tails    = double(ceilDiv(ceilDiv(tail_tiles, cus), uint64_t(vi.occupancy)));
     const double compute  = double(per_cu) * (flops / double(tiles)) / cu_rate + rounds * kRoundMicros +
