@@ -127,8 +127,9 @@ def test_fp32_unaligned_in_place(capi, ops):
 @pytest.mark.parametrize("kind,cd", [("bf16", "fp32"), ("fp16", "fp16")])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 def test_half_unaligned_tiles(capi, ops, kind, cd, ta, tb):
-    for m, n, k in ((129, 131, 257), (128, 128, 259), (255, 257, 319), (300, 129, 383), (131, 300, 320), (65, 66, 100),
-                    (127, 127, 300), (66, 500, 333), (1500, 1601, 129)):
+    for m, n, k in ((129, 131, 1281), (128, 128, 1283), (255, 257, 1151), (255, 257, 1215), (300, 129, 1407),
+                    (131, 300, 1344), (65, 66, 100), (127, 127, 1300), (66, 500, 1357), (300, 129, 639), (131, 300, 641),
+                    (1500, 1601, 385)):
         for with_c, ab_pad, ab_shift, cd_pad in ((True, 0, 0, 0), (False, 3, 1, 1), (True, 1, 5, 3)):
             names = check(capi, ops, kind, cd, m, n, k, ta, tb, with_c, ab_pad, ab_shift, cd_pad, 1 if cd_pad else 0,
                           only="Unaligned")
@@ -137,8 +138,8 @@ def test_half_unaligned_tiles(capi, ops, kind, cd, ta, tb):
 
 def test_half_unaligned_in_place(capi, ops):
     # c and d one matrix: the outputs that a moved last tile shares with its neighbour are written once.
-    a = torch.randint(-4, 5, (300, 301), device="cuda").bfloat16()
-    b = torch.randint(-4, 5, (301, 301), device="cuda").bfloat16()
+    a = torch.randint(-4, 5, (300, 1325), device="cuda").bfloat16()
+    b = torch.randint(-4, 5, (1325, 301), device="cuda").bfloat16()
     c = torch.randint(-4, 5, (300, 301), device="cuda").float()
     want = (0.5 * (a.double() @ b.double()) + 2.0 * c.double()).float()
     d = c.clone()
