@@ -5,7 +5,8 @@
 // d = alpha * (a @ b) + beta * c, the contract of the other 16-bit tiles (fp32 accumulation; c and d
 // in fp32 or the input type; with a null c the beta term is dropped).  Applicability, checked on the
 // host, is that of the DMA tiles of dma_tile.hpp (16-byte aligned a and b, leading dimensions
-// multiples of 8 and below 2^23, those of c and d below 2^21); m, n and k are free.
+// multiples of 8 and below 2^23, those of c and d below 2^21, a's and b's contiguous extents multiples
+// of 8); m, n and k are free otherwise.
 //
 // Workgroup: 8 waves, two per SIMD.  Wave w is in group wm = w / 4 and has column place wn = w % 4.
 // The tile's rows come in two halves of 128, its columns too; a wave owns, of each of the four
@@ -40,7 +41,7 @@
 // SIMD that alternate lose almost none, 16x16x32 MFMAs draw less power per FLOP, and the longer DMA
 // lead covers HBM, so a b larger than the last-level cache needs no prefetch.  Measured on MI355X
 // against that tile, same box, bf16, us: 16384x14336x4096 with column-major b and 16-bit d 1577 ->
-// 1256, 4096x4096x8200 with column-major a 219 -> 185, 2048x114688x4096 1526 -> 1411, grouped
+// 1256, 4096x4096x8200 with column-major a and fp32 c 219 -> 199, 2048x114688x4096 1526 -> 1411, grouped
 // 16384x14336x4096 over 8 / 64 experts 1680 -> 1503 / 2599 -> 2396.  Phases of 16 MFMAs instead of 32
 // (barriers twice as often, LDS reads and waits no longer covered) ran 10% slower (8192^3 826 against
 // 757); raising the wave priority in the matrix part was 0.5% slower, DMAs before the reads the same.
@@ -418,15 +419,20 @@ __device__ __forceinline__ void half_gemm_pp_tile(const HalfGemmParams& p, int b
         }
     }
 
-    // Epilogue.  Lane (j16, g) holds row j16, columns 4 g .. 4 g + 3 of every block.  Buffer accesses
-    // relative to the tile's corner: the lane part of the offset in the VGPR offset, the block part in
-    // the scalar offset.  An element outside the matrix gets the lane offset 2^31, past the buffer's
-    // size (at most 2^31 - 1 bytes), so its c load returns 0 and its store is dropped; ldc and ldd
-    // below 2^21 keep every sum below 2^32.
-    //   WIDE (n, ldc, ldd multiples of 8 elements' worth of 16 bytes and c, d aligned): fp32 d in
-    // 16-byte stores, 4 lanes covering 64 bytes of a row; 16-bit d packs two neighbouring blocks'
-    // 8 bytes and exchanges odd and even lane groups (v_permlane16_swap), after which a lane holds 8
-    // adjacent columns: again 16 bytes per lane and 64 per row.  Otherwise element by element.
+    // Epilogue.  Lane (j16, g) holds row j16, columns 4 g .. 4 g + 3 of every 16x16 block; stored from
+    // there, every access would touch 16 rows.  One row half of the tile at a time is therefore turned
+    // over through LDS (128 rows of 1 KiB, 16-byte chunk c of row r at slot c ^ (r & 15): neither side
+    // has bank conflicts), after which a wave owns 16 whole rows: an access covers one row of 1 KiB in
+    // fp32, two of 512 bytes in 16 bits.  c is loaded in that layout, a row half ahead of its use.
+    //   Buffer accesses relative to the tile's corner: the lane part of the offset in the VGPR offset, the
+    // row in the scalar offset.  An element outside the matrix gets the lane offset 2^31, past the
+    // buffer's size (at most 2^31 - 1 bytes), so its c load returns 0 and its store is dropped; ldc and
+    // ldd below 2^21 keep every sum below 2^32.  A buffer access of 16 bytes needs an address aligned to 4:
+    // 16-bit c and d whose rows are not (!WIDE) take global accesses, which need no alignment.  The chunk
+    // across the last column, if there is one, goes element by element.
+    //   Measured against stores from the MFMA layout (16 rows of 64 bytes per access; element by element
+    // where n, ldc or ldd were not multiples of 16 bytes), fp16, us: 9216x2827x2112 with a column-major b
+    // and 16-bit d 275 -> 115; bf16 with c, 8192x8192x256 114 -> 92, 3584x6272x512 (fp32 c) 69 -> 60.
     const float alpha = p.alpha, beta = p.beta;
     const unsigned ldd = static_cast<unsigned>(p.ldd), ldc = static_cast<unsigned>(p.ldc);
     const int rows_left = M - m0, cols_left = N - n0;
@@ -434,125 +440,131 @@ __device__ __forceinline__ void half_gemm_pp_tile(const HalfGemmParams& p, int b
     auto epilogue = [&](auto c_tag, auto half_tag, auto wide_tag) {
         constexpr bool HAS_C = decltype(c_tag)::value, HALF = decltype(half_tag)::value, WIDE = decltype(wide_tag)::value;
         constexpr unsigned ES = HALF ? 2 : 4;
+        constexpr int EPL = HALF ? 8 : 4, RPA = HALF ? 2 : 1;  // elements per lane, rows per access
+        constexpr int NA = 16 / RPA;                           // accesses of a wave per row half
         // 16-bit d is stored non-temporal (2), fp32 d is not (0): measured, above.
         constexpr int kPolicy = HALF ? 2 : 0;
+        typedef u32x4 u32x4_any __attribute__((aligned(2)));
+        const int er = HALF ? lane >> 5 : 0, ec = EPL * (HALF ? lane & 31 : lane);
+        const bool full = ec + EPL <= cols_left, cut = ec < cols_left && !full;
+        const bool any_cut = cols_left < 256 && cols_left % EPL != 0;
         auto span = [&](uint64_t ld) {
             const uint64_t b = ((uint64_t)(rows_left - 1) * ld + (uint64_t)cols_left) * ES;
             return static_cast<int>(b < 0x7FFFFFFFull ? b : 0x7FFFFFFFull);
         };
-        const __amdgpu_buffer_rsrc_t dres = __builtin_amdgcn_make_buffer_rsrc(
-            static_cast<char*>(p.d) + ((size_t)m0 * p.ldd + n0) * ES, 0, span(p.ldd), kBufferConfig);
+        char* const dcorner = static_cast<char*>(p.d) + ((size_t)m0 * p.ldd + n0) * ES;
+        const __amdgpu_buffer_rsrc_t dres = __builtin_amdgcn_make_buffer_rsrc(dcorner, 0, span(p.ldd), kBufferConfig);
+        const char* ccorner         = nullptr;
         __amdgpu_buffer_rsrc_t cres = dres;
-        if constexpr (HAS_C)
-            cres = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<char*>(static_cast<const char*>(p.c)) + ((size_t)m0 * p.ldc + n0) * ES, 0, span(p.ldc),
-                kBufferConfig);
+        if constexpr (HAS_C) {
+            ccorner = static_cast<const char*>(p.c) + ((size_t)m0 * p.ldc + n0) * ES;
+            cres    = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(ccorner), 0, span(p.ldc), kBufferConfig);
+        }
+        const unsigned lane_d = (er * ldd + ec) * ES, lane_c = (er * ldc + ec) * ES;
+        auto row_of = [&](int i, int t) { return 128 * i + 16 * wave + RPA * t; };  // wave-uniform
+        u32x4 cv[HAS_C ? NA : 1];
+        auto load_c = [&](int i, int t) {
+            if constexpr (HAS_C) {
+                const int row0 = row_of(i, t);
+                const bool ok  = full && row0 + er < rows_left;
+                if constexpr (HALF && !WIDE) {
+                    cv[t] = u32x4{0u, 0u, 0u, 0u};
+                    if (ok) cv[t] = *reinterpret_cast<const u32x4_any*>(ccorner + (size_t)(row0 * ldc) * ES + lane_c);
+                } else {
+                    cv[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                          cres, ok ? lane_c : kOut, static_cast<int>(row0 * ldc * ES), 0));
+                }
+            }
+        };
+        auto element = [&](const u32x4& w, int e) {
+            if constexpr (HALF)
+                return to_float<BF16>(static_cast<u16>(w[e >> 1] >> (16 * (e & 1))));
+            else
+                return __builtin_bit_cast(floatx4, w)[e];
+        };
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int t = 0; t < NA; ++t) load_c(0, t);
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+        for (int i = 0; i < 2; ++i) {
+            if (128 * i >= rows_left) break;
+            // The other waves are done with what LDS held.
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int row0   = 128 * i + 64 * wm + 16 * u;  // wave-uniform
-                    const int col0   = 128 * j + 32 * wn;
-                    const bool rowok = row0 + j16 < rows_left;
-                    float out[2][4];
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int v = 0; v < 2; ++v) {
-                        const int cc = col0 + 16 * v;
-                        float cv[4] = {0.f, 0.f, 0.f, 0.f};
-                        if constexpr (HAS_C) {
-                            const unsigned lane_c = (j16 * ldc + 4 * g) * ES;
-                            const int so = static_cast<int>((row0 * ldc + cc) * ES);
-                            if constexpr (WIDE) {
-                                const unsigned off = rowok && cc + 4 * g < cols_left ? lane_c : kOut;
-                                if constexpr (HALF) {
-                                    const u32x2 w = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(cres, off, so, 0));
+                for (int u = 0; u < 4; ++u)
 #pragma unroll
-                                    for (int e = 0; e < 4; ++e) cv[e] = to_float<BF16>(static_cast<u16>(w[e >> 1] >> (16 * (e & 1))));
-                                } else {
-                                    const floatx4 w = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(cres, off, so, 0));
+                    for (int v = 0; v < 2; ++v)
+                        *reinterpret_cast<floatx4*>(lds + (64 * wm + 16 * u + j16) * 1024 +
+                                                    16 * ((32 * j + 8 * wn + 4 * v + g) ^ j16)) = alpha * acc[i][j][u][v];
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-                                    for (int e = 0; e < 4; ++e) cv[e] = w[e];
-                                }
+            for (int t = 0; t < NA; ++t) {
+                const int row0 = row_of(i, t), r = 16 * wave + RPA * t + er;
+                float out[EPL];
+#pragma unroll
+                for (int q = 0; q < EPL / 4; ++q) {
+                    const floatx4 f = *reinterpret_cast<const floatx4*>(lds + r * 1024 + 16 * ((ec / 4 + q) ^ (r & 15)));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) out[4 * q + e] = f[e];
+                }
+                if (any_cut) {
+                    if (cut && row0 + er < rows_left) {
+                        const size_t at_d = ((size_t)(row0 + er) * ldd + ec) * ES, at_c = ((size_t)(row0 + er) * ldc + ec) * ES;
+#pragma unroll
+                        for (int e = 0; e < EPL - 1; ++e) {
+                            if (ec + e >= cols_left) break;
+                            float x = out[e];
+                            if constexpr (HALF) {
+                                if constexpr (HAS_C) x += beta * to_float<BF16>(reinterpret_cast<const u16*>(ccorner + at_c)[e]);
+                                reinterpret_cast<u16*>(dcorner + at_d)[e] = from_float<BF16>(x);
                             } else {
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) {
-                                    const unsigned off = rowok && cc + 4 * g + e < cols_left ? lane_c + e * ES : kOut;
-                                    if constexpr (HALF)
-                                        cv[e] = to_float<BF16>(static_cast<u16>(__builtin_amdgcn_raw_buffer_load_b16(cres, off, so, 0)));
-                                    else
-                                        cv[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(cres, off, so, 0));
-                                }
-                            }
-                        }
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            out[v][e] = alpha * acc[i][j][u][v][e];
-                            if constexpr (HAS_C) out[v][e] += beta * cv[e];
-                        }
-                    }
-                                    if constexpr (WIDE && HALF) {
-                        unsigned x0 = pack2<BF16>(out[0][0], out[0][1]), x1 = pack2<BF16>(out[0][2], out[0][3]);
-                        unsigned y0 = pack2<BF16>(out[1][0], out[1][1]), y1 = pack2<BF16>(out[1][2], out[1][3]);
-                        // Odd lane groups of x change places with even ones of y: groups 0 and 2 then
-                        // hold columns 4 g .. 4 g + 7 of block 0, groups 1 and 3 columns 4 (g - 1) .. of
-                        // block 1.
-                        const auto s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);
-                        const auto s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
-                        const u32x4 w{s0[0], s1[0], s0[1], s1[1]};
-                        const int lc = 16 * (g & 1) + 4 * (g & 2);
-                        const unsigned lane_d = (j16 * ldd + lc) * ES;
-                        const unsigned off    = rowok && col0 + lc < cols_left ? lane_d : kOut;
-                        __builtin_amdgcn_raw_buffer_store_b128(w, dres, off, static_cast<int>((row0 * ldd + col0) * ES), kPolicy);
-                        asm volatile("s_nop 1" ::"v"(w) : "memory");
-                    } else {
-                        const unsigned lane_d = (j16 * ldd + 4 * g) * ES;
-#pragma unroll
-                        for (int v = 0; v < 2; ++v) {
-                            const int cc = col0 + 16 * v;
-                            const int so = static_cast<int>((row0 * ldd + cc) * ES);
-                            if constexpr (WIDE) {
-                                const floatx4 f{out[v][0], out[v][1], out[v][2], out[v][3]};
-                                const u32x4 w = __builtin_bit_cast(u32x4, f);
-                                __builtin_amdgcn_raw_buffer_store_b128(w, dres, rowok && cc + 4 * g < cols_left ? lane_d : kOut, so, kPolicy);
-                                // The data registers stay unwritten for two wait states after the
-                                // store (a VALU write right after it has replaced its first dword).
-                                asm volatile("s_nop 1" ::"v"(w) : "memory");
-                            } else {
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) {
-                                    const unsigned off = rowok && cc + 4 * g + e < cols_left ? lane_d + e * ES : kOut;
-                                    if constexpr (HALF)
-                                        __builtin_amdgcn_raw_buffer_store_b16(from_float<BF16>(out[v][e]), dres, off, so, kPolicy);
-                                    else
-                                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, out[v][e]), dres, off, so, kPolicy);
-                                }
+                                if constexpr (HAS_C) x += beta * reinterpret_cast<const float*>(ccorner + at_c)[e];
+                                reinterpret_cast<float*>(dcorner + at_d)[e] = x;
                             }
                         }
                     }
                 }
+                if constexpr (HAS_C) {
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e) out[e] += beta * element(cv[t], e);
+                    if (i == 0) load_c(1, t);
+                }
+                u32x4 w;
+                if constexpr (HALF)
+                    w = u32x4{pack2<BF16>(out[0], out[1]), pack2<BF16>(out[2], out[3]), pack2<BF16>(out[4], out[5]),
+                              pack2<BF16>(out[6], out[7])};
+                else
+                    w = __builtin_bit_cast(u32x4, floatx4{out[0], out[1], out[2], out[3]});
+                const bool ok = full && row0 + er < rows_left;
+                if constexpr (HALF && !WIDE) {
+                    if (ok) *reinterpret_cast<u32x4_any*>(dcorner + (size_t)(row0 * ldd) * ES + lane_d) = w;
+                } else {
+                    __builtin_amdgcn_raw_buffer_store_b128(w, dres, ok ? lane_d : kOut, static_cast<int>(row0 * ldd * ES), kPolicy);
+                    // The data registers stay unwritten for two wait states after the store (a VALU write
+                    // right after it has replaced its first dword).
+                    asm volatile("s_nop 1" ::"v"(w) : "memory");
+                }
+            }
+        }
     };
-    auto with_wide = [&](auto c_tag, auto half_tag) {
-        const unsigned unit = p.cd_half ? 8 : 4;  // elements of 16 bytes
-        const bool wide = N % unit == 0 && ldd % unit == 0 && (uintptr_t)p.d % 16 == 0 &&
-                          (p.c == nullptr || (ldc % unit == 0 && (uintptr_t)p.c % 16 == 0));
+    auto with_half = [&](auto c_tag) {
+        if (!p.cd_half) {
+            epilogue(c_tag, std::false_type{}, std::true_type{});
+            return;
+        }
+        // Every row of c and d on a 4-byte address.
+        const bool wide = ldd % 2 == 0 && (uintptr_t)p.d % 4 == 0 &&
+                          (p.c == nullptr || (ldc % 2 == 0 && (uintptr_t)p.c % 4 == 0));
         if (wide)
-            epilogue(c_tag, half_tag, std::true_type{});
+            epilogue(c_tag, std::true_type{}, std::true_type{});
         else
-            epilogue(c_tag, half_tag, std::false_type{});
+            epilogue(c_tag, std::true_type{}, std::false_type{});
     };
-    if (p.c != nullptr) {
-        if (p.cd_half)
-            with_wide(std::true_type{}, std::true_type{});
-        else
-            with_wide(std::true_type{}, std::false_type{});
-    } else {
-        if (p.cd_half)
-            with_wide(std::false_type{}, std::true_type{});
-        else
-            with_wide(std::false_type{}, std::false_type{});
-    }
+    if (p.c != nullptr)
+        with_half(std::true_type{});
+    else
+        with_half(std::false_type{});
 }
 
 // Tile rows walked as one band (tile_of).

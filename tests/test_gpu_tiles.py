@@ -86,6 +86,54 @@ def test_half_tile_edges(capi, ops, kind, cd, ta, tb):
         check(capi, ops, kind, cd, 264, 130, 1032, ta, tb, True)
 
 
+def us_of(run, reps=20, rounds=5):
+    """Median microseconds of a launch among others."""
+    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    got = []
+    for _ in range(rounds + 1):
+        start.record()
+        for _ in range(reps):
+            run()
+        stop.record()
+        torch.cuda.synchronize()
+        got.append(start.elapsed_time(stop) / reps * 1e3)
+    return sorted(got[1:])[rounds // 2]
+
+
+def tile_us(capi, ops, name, dtype, out, m, n, k, tb, with_c):
+    a = torch.zeros(m, k, dtype=dtype, device="cuda")
+    b = torch.zeros(n, k, dtype=dtype, device="cuda").t() if tb else torch.zeros(k, n, dtype=dtype, device="cuda")
+    c = torch.zeros(m, n, dtype=out, device="cuda") if with_c else None
+    d = torch.empty(m, n, dtype=out, device="cuda")
+    plan = capi.plan_for(a, b, c, d, 1.0, 0.5 if with_c else 0.0, ops)
+    i = plan.names().index(name)
+    return us_of(lambda: plan.execute(i, torch.cuda.current_stream().cuda_stream))
+
+
+# Rows of d that start on odd 2-byte addresses: a tile's stores stay whole rows.  The two launches differ by
+# the 5 columns (under 1%); stores of single elements took 2.6 times as long.
+@pytest.mark.parametrize("with_c", [False, True])
+def test_half_256_tile_cost_of_unaligned_rows(capi, ops, with_c):
+    odd, even = (tile_us(capi, ops, "Fp16MfmaGemm_256x256_Dma", torch.float16, torch.float16, 4096, n, 1024, True, with_c)
+                 for n in (2811, 2816))
+    assert odd < 1.6 * even, (odd, even)
+
+
+def test_half_256_tile_in_place(capi, ops):
+    # c and d one matrix, rows on odd addresses and a last tile of 1 to 7 columns past a multiple of 8.
+    for n, out in ((257, torch.float32), (262, torch.bfloat16), (519, torch.bfloat16)):
+        a = torch.randint(-4, 5, (300, 136), device="cuda").bfloat16()
+        b = torch.randint(-4, 5, (n, 136), device="cuda").bfloat16().t()
+        c = torch.randint(-4, 5, (300, n), device="cuda").to(out)
+        want = (0.5 * (a.double() @ b.double()) + 2.0 * c.double()).float().to(out)
+        d = c.clone()
+        plan = capi.plan_for(a, b, d, d, 0.5, 2.0, ops)
+        i = plan.names().index("Bf16MfmaGemm_256x256_Dma")
+        plan.execute(i, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(d, want), (n, out)
+
+
 # Launches of at most one workgroup per CU (three stage buffers) and of more, 1 to 7 stages, whole-k.
 @pytest.mark.parametrize("m,n", [(128, 128), (2048, 2048), (2048, 2176)])
 def test_half_128_tile_stage_counts(capi, ops, m, n):
