@@ -250,12 +250,16 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
         const int64_t b_rs = g.tb ? 1 : g.ldb, b_cs = g.tb ? g.ldb : 1;
         wide_ = WideParams{a, b, c, d, alpha, beta, s.m, s.n, s.k, a_rs, a_cs, b_rs, b_cs, g.ldc, g.ldd};
 
-        int threads = info_->threads;
-        kernel_     = info_->gemv && info_->split == SplitKind::kNone ? gemm::gemvKernel(v_, int(s.m), g.ta, g.tb, threads)
-                                                                  : gemm::kernelFor(v_, g.ta, g.tb);
-        checkBlockSize(kernel_, threads, info_->name);
-        block_  = dim3(threads);
+        // The kernel the launch runs, whichever form of the variant that is, with its workgroup size.
+        const auto use = [&](const void* kernel, int threads) {
+            if (kernel == nullptr)
+                raise(FTRAIN_STATUS_INTERNAL_ERROR, "%s: no kernel for these operand orientations", info_->name);
+            checkBlockSize(kernel, threads, info_->name);
+            kernel_ = kernel;
+            block_  = dim3(threads);
+        };
         if (info_->simt) {
+            use(gemm::kernelFor(v_, g.ta, g.tb), info_->threads);
             const uint64_t tiles = ceilDiv(s.m, 64) * ceilDiv(s.n, 64);
             grid_                = dim3(static_cast<uint32_t>(std::min<uint64_t>(tiles, 1u << 20)));
             return;
@@ -277,7 +281,11 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
                                       0,            0,            g.lda,        g.ldb, g.ldc, g.ldd,
                                       int32_t(cd_half)};
         if (info_->gemv) {
-            grid_ = dim3(static_cast<uint32_t>(ceilDiv(s.n, uint64_t(info_->bn))), 1, splits);
+            grid_              = dim3(static_cast<uint32_t>(ceilDiv(s.n, uint64_t(info_->bn))), 1, splits);
+            int threads        = info_->threads;
+            const void* kernel = info_->split == SplitKind::kNone ? gemm::gemvKernel(v_, int(s.m), g.ta, g.tb, threads)
+                                                                  : gemm::kernelFor(v_, g.ta, g.tb);
+            use(kernel, threads);
         } else {
             params_.tiles_m = half_params_.tiles_m = int32_t(ceilDiv(s.m, info_->bm));
             params_.tiles_n = half_params_.tiles_n = int32_t(ceilDiv(s.n, info_->bn));
@@ -287,11 +295,11 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
                 half_params_.tiles_m = int32_t(ceilDiv(s.m, 128));
                 half_params_.tiles_n = int32_t(ceilDiv(s.n, 128));
                 grid_   = dim3(uint32_t(half_params_.tiles_m) * uint32_t(half_params_.tiles_n));
-                kernel_ = gemm::halfUnaligned128(v_ == Variant::kBf16Mfma64x64U, g.ta, g.tb);
+                use(gemm::halfUnaligned128(v_ == Variant::kBf16Mfma64x64U, g.ta, g.tb), info_->threads);
                 return;
             }
-            unsplit_        = splits == 1 && gemm::unsplitForm(v_);
-            kernel_         = gemm::kernelFor(v_, g.ta, g.tb, uint64_t(grid_.x) * splits <= uint64_t(cus), unsplit_);
+            unsplit_ = splits == 1 && gemm::unsplitForm(v_);
+            use(gemm::kernelFor(v_, g.ta, g.tb, uint64_t(grid_.x) * splits <= uint64_t(cus), unsplit_), info_->threads);
         }
         const uint64_t count = s.m * s.n;
         if (info_->split == SplitKind::kFused) {
