@@ -59,6 +59,10 @@ constexpr double kThinRoundMicros = 7.0;  // a second round on few CUs, see mode
 // weight from memory (MLP forward over 8 experts 0.53 of peak, plain 0.58-0.62).
 constexpr double kGroupedHalf256Efficiency = 0.66;
 constexpr double kTieWeight       = 1e-3;
+// The skinny kernel for a column-major b with five rows or more: bytes per microsecond over its rounds of
+// one workgroup per CU, and a fixed cost.
+constexpr double kGemvManyRowsRate   = 5.6e6;
+constexpr double kGemvManyRowsMicros = 2.0;
 constexpr double kCuBytesPerMicro = 6.4e4;  // one CU's sustained load rate (about 27 bytes per clock)
 // A DMA tile stages a partial last stage (k not a multiple of its stage) by ordinary loads once its
 // pipeline has drained: per tile, the drain, the loads' latency and a barrier.  Fitted to the bf16
@@ -125,7 +129,8 @@ double residentEfficiency(const VariantInfo& vi, uint64_t per_cu) {
 }
 
 // Modelled time of variant `v` with a given split count (1 = no split).
-double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cus, uint64_t splits) {
+double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cus, uint64_t splits,
+                   const OperandForm& o = {}) {
     const double m = double(s.m), n = double(s.n), k = double(s.k);
     // a and b in the variant's input type; c and d counted at the same size.
     const double eb   = vi.input == FTRAIN_NUMERIC_TYPE_FP32 ? 4.0 : 2.0;
@@ -152,10 +157,16 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
         // 5.4-6.3 TB/s, 256 waves lose to split-k).
         // A CU also loads at a bounded rate, so a launch of few workgroups is bound by the bytes each
         // one reads (bf16 1x4096x4096, 64 workgroups of 512 KiB: 9.0 us).
-        const int threads = vi.split == SplitKind::kNone ? gemvPassThreads(int(std::max<uint64_t>(s.m, 1))) : vi.threads;
+        const int threads = vi.split == SplitKind::kNone ? gemvPassThreads(int(std::max<uint64_t>(s.m, 1)), o.tb) : vi.threads;
         const double wgs  = double(ceilDiv(std::max<uint64_t>(s.n, 1), uint64_t(vi.bn)) * splits);
         const double fill = std::min(1.0, wgs * (threads / 64) / (double(cus) * 4.0));
         const double per_cu = std::ceil(wgs / double(cus)) * bytes / wgs;
+        // From five rows on, the form for a column-major b has room for one workgroup per CU: a last round
+        // on few CUs takes as long as a full one (us, against the best split tile: 8x8192x8192, 256
+        // workgroups, 58.7 / 74.9; 7x12768x4600, 399, 50 / 64; 5x8824x13680, 276, 183 / 127; 6x11688x12376,
+        // 366, 174 / 147; 5x9864x2488, 309, 41 / 34).
+        if (o.tb && vi.split == SplitKind::kNone && s.m > 4)
+            return std::ceil(wgs / double(cus)) * double(cus) / wgs * bytes / kGemvManyRowsRate + kGemvManyRowsMicros + launch;
         const double t      = std::max(bytes / (kHbmBytesPerMicro * fill), per_cu / kCuBytesPerMicro) + serial_us + launch;
         // The split-k skinny kernel keeps few loads in flight per wave and runs well below the
         // streaming model, more so with more rows of a (measured on MI355X, us, model in brackets:
@@ -293,12 +304,12 @@ uint32_t chooseSplits(Variant v, const GemmShape& s, int cus) {
     return static_cast<uint32_t>(best);
 }
 
-double estimateMicros(Variant v, const GemmShape& s, bool has_c, int cus) {
+double estimateMicros(Variant v, const GemmShape& s, bool has_c, int cus, const OperandForm& o) {
     const VariantInfo& vi = info(v);
     if (vi.gemv && s.m > uint64_t(vi.bm)) return std::numeric_limits<double>::infinity();
     const uint32_t splits = vi.split != SplitKind::kNone ? chooseSplits(v, s, cus) : 1;
     if (splits == 0) return std::numeric_limits<double>::infinity();
-    return modelMicros(vi, s, has_c, cus, splits);
+    return modelMicros(vi, s, has_c, cus, splits, o);
 }
 
 double groupedMicros(Variant v, const std::vector<GemmShape>& shapes, bool has_c, int cus) {
@@ -334,14 +345,17 @@ double groupedMicros(Variant v, const std::vector<GemmShape>& shapes, bool has_c
 std::vector<std::string> ShapeCostFinder::candidates(const GemmProblem& problem, const Constraints& constraints) {
     // Rank on the shape the kernels run: a column-major d swaps m and n.
     GemmLaunch g;
-    const GemmShape s = problem.launch(g) == nullptr ? g.shape : problem.shape();
+    const bool runs   = problem.launch(g) == nullptr;
+    const GemmShape s = runs ? g.shape : problem.shape();
     const int cus     = gemm::computeUnits(constraints.device());
     const bool has_c  = problem.c().memory() != nullptr;
+    gemm::OperandForm o;
+    if (runs) o.tb = g.tb;
     std::vector<std::pair<double, int>> ranked;
     for (int i = 0; i < static_cast<int>(gemm::Variant::kCount); ++i) {
         // Only variants for a's element type compete.
         if (gemm::info(static_cast<gemm::Variant>(i)).input != problem.a().numericType()) continue;
-        const double t = gemm::estimateMicros(static_cast<gemm::Variant>(i), s, has_c, cus);
+        const double t = gemm::estimateMicros(static_cast<gemm::Variant>(i), s, has_c, cus, o);
         if (std::isfinite(t)) ranked.emplace_back(t, i);
     }
     std::stable_sort(ranked.begin(), ranked.end(),

@@ -486,13 +486,12 @@ __global__ __launch_bounds__(256) void simt_gemm(WideParams p) {
 // one row 8 waves x 2 steps (37.8 us), two and four rows 16 x 2 (38.9 /
 // 38.8), eight rows 8 x 2 (the configurations with more in flight, 8 x 4
 // and 16 x 2, spill registers there).  The 16-bit kernel uses the same.
-int gemvPassThreads(int m) { return m <= 1 || m > 4 ? 512 : 1024; }
+int gemvPassThreads(int m, bool tb) { return tb || m <= 1 || m > 4 ? 512 : 1024; }
 
 const void* gemvKernel(Variant v, int m, bool ta, bool tb, int& threads) {
-    threads = gemvPassThreads(m);
+    threads = gemvPassThreads(m, tb);
     if (v == Variant::kBf16Gemv || v == Variant::kFp16Gemv) return ta || tb ? nullptr : gemvHalfKernel(v == Variant::kBf16Gemv, m);
     if (tb) {
-        threads = 512;
         if (ta) return nullptr;
         if (m <= 1) return reinterpret_cast<const void*>(&gemv_pass_tb<4, 1>);
         if (m <= 2) return reinterpret_cast<const void*>(&gemv_pass_tb<4, 2>);

@@ -222,7 +222,8 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
         // one row 8192^2 44.7 / 73.2, 14336x4096 42.7 / 65.5, 2048^2 6.0 / 10.4; two rows 45.8 / 73.8, 45.8 /
         // 65.8, 7.1 / 10.5; four rows 8192^2 49.1 / 74.5, 1024^2 6.1 / 9.6, but 4096x14336 75 / 62; eight rows
         // 8192^2 58.7 / 74.9, but 4096x8192 51.9 / 42.2 (n x k).
-        if (v_ == Variant::kGemv && g.tb && s.m > 2 && s.n < 8192 && (s.m > 4 || s.k > 2048))
+        if (v_ == Variant::kGemv && g.tb && s.m > 2 && (s.m > 4 || s.k > 2048) &&
+            ceilDiv(s.n, uint64_t(info_->bn)) < uint64_t(gemm::computeUnits(constraints.device())))
             return Result(FTRAIN_STATUS_UNSUPPORTED, "too few columns of a column-major b for this many rows (skinny kernel)");
         if (info_->split == SplitKind::kPartial &&
             gemm::chooseSplits(v_, s, gemm::computeUnits(constraints.device())) == 0)

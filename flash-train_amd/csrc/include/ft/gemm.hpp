@@ -125,8 +125,13 @@ uint32_t chooseSplits(Variant v, const GemmShape& s, int cus);
 // restores the model.  Process-wide.
 void forceSplits(uint32_t s);
 
+// What the cost model takes of a problem's operands beside their sizes.
+struct OperandForm {
+    bool tb = false;  // column-major b
+};
+
 // Modelled execution time in microseconds (lower is better).
-double estimateMicros(Variant v, const GemmShape& s, bool has_c, int cus);
+double estimateMicros(Variant v, const GemmShape& s, bool has_c, int cus, const OperandForm& o = {});
 
 // Compute units of `device` (cached; 256 when HIP cannot be queried).
 int computeUnits(FTrainDeviceId device);

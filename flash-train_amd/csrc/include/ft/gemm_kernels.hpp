@@ -281,9 +281,9 @@ bool unsplitForm(Variant v);
 // The one-pass skinny kernels (Variant::kGemv, kBf16Gemv, kFp16Gemv) for m
 // rows of a (up to the variant's row limit) and a row-major (ta false) or,
 // fp32 only, column-major a; null otherwise.  `threads` receives the
-// workgroup size.  b is row-major (gemvPassThreads(m) threads) or, fp32 with a row-major a only,
-// column-major (512).
-int gemvPassThreads(int m);
+// workgroup size, gemvPassThreads(m, tb).  b is row-major or, fp32 with a row-major a only,
+// column-major.
+int gemvPassThreads(int m, bool tb);
 const void* gemvKernel(Variant v, int m, bool ta, bool tb, int& threads);
 const void* gemvHalfKernel(bool bf16, int m);
 // Per-layout instantiations of the layout-capable MFMA variants (one HIP TU

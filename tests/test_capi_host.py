@@ -577,10 +577,12 @@ def test_zero_depth_needs_no_a_or_b(tlib, tops):
 # ------------------------------------------------------------------ Finder choices
 
 
-def rank(tlib, m, n, k, addr=FAKE, with_c=False, device=0, ab_type=c.FP32):
+def rank(tlib, m, n, k, addr=FAKE, with_c=False, device=0, ab_type=c.FP32, cd_type=c.FP32, tb=False):
     views = (c.StorageView * 6)()
-    keep = [V([m, k], addr, numeric_type=ab_type), V([k, n], addr, numeric_type=ab_type),
-            V([m, n], addr if with_c else None), V([m, n], addr)]
+    b = V([k, n], addr, numeric_type=ab_type) if not tb else V([k, n], addr, numeric_type=ab_type,
+                                                               index_type=c.INDEX_INVALID, strides=[1, k])
+    keep = [V([m, k], addr, numeric_type=ab_type), b, V([m, n], addr if with_c else None, numeric_type=cd_type),
+            V([m, n], addr, numeric_type=cd_type)]
     al, be = c.HostScalar(1.0), c.HostScalar(0.0)
     for i, v in enumerate(keep + [al.view, be.view]):
         views[i] = v.sv
@@ -632,6 +634,16 @@ def test_finder_choices_for_the_baseline_configs(tlib):
     # Odd sizes: no 128-bit variant applies.
     odd = rank(tlib, 127, 97, 33)
     assert odd and all(("Unaligned" in n) or n == "Fp32Gemm" for n in odd)
+
+
+def test_finder_choices_for_a_skinny_column_major_b(tlib):
+    # us on the skinny kernel and on the fastest split tile (copies that do not fit the last-level cache): it wins
+    # with one or two rows, and with more only where its workgroups of 32 columns fill their rounds of the 256 CUs.
+    for m, n, k, skinny, tile in ((1, 8192, 8192, 44.7, 73.2), (2, 6832, 2520, 13.5, 26.0), (4, 12304, 3064, 34.0, 48.6),
+                                  (8, 8192, 8192, 58.7, 74.9), (7, 12768, 4600, 49.7, 66), (5, 8824, 13680, 183, 127),
+                                  (6, 11688, 12376, 174, 147), (5, 9476, 7912, 101, 81)):
+        first = rank(tlib, m, n, k, tb=True)[0]
+        assert (first == "Fp32Gemv") == (skinny < tile), (m, n, k, first)
 
 
 def test_finder_choices_for_16_bit_skinny_m(tlib):
