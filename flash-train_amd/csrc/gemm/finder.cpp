@@ -59,6 +59,11 @@ constexpr double kThinRoundMicros = 7.0;  // a second round on few CUs, see mode
 // weight from memory (MLP forward over 8 experts 0.53 of peak, plain 0.58-0.62).
 constexpr double kGroupedHalf256Efficiency = 0.66;
 constexpr double kTieWeight       = 1e-3;
+// The whole-k form of the fp32 64x64 split tile, see modelMicros: its rate on rows of part lines, and of one
+// workgroup per CU on operands larger than the L2s (8 of 4 MiB).
+constexpr double kWholePartLines = 0.95;
+constexpr double kWholeStreaming = 0.72;
+constexpr double kL2Bytes        = 32.0 * 1048576.0;
 // The skinny kernel for a column-major b with five rows or more: bytes per microsecond over its rounds of
 // one workgroup per CU, and a fixed cost.
 constexpr double kGemvManyRowsRate   = 5.6e6;
@@ -187,7 +192,16 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
     const uint64_t per_cu  = ceilDiv(wgs, cus);
     const double depth     = double(std::max<uint64_t>(chunk, vi.bk));
     // SIMT FMAs run at half the matrix rate without packed FP32.
-    const double cu_rate   = vi.flop_per_clk * kClockPerMicro * residentEfficiency(vi, per_cu) * (vi.simt ? 0.5 : 1.0);
+    double cu_rate         = vi.flop_per_clk * kClockPerMicro * residentEfficiency(vi, per_cu) * (vi.simt ? 0.5 : 1.0);
+    // The whole-k form of the fp32 64x64 split tile loads twice what the 128x128 tile does per FLOP.  Rows
+    // that are not whole 128-byte lines cost it more (us, against 128x128 whole-k or split: 3652x12080x7296
+    // 4760 / 4410, 9584x4124x7564 4380 / 4180, 2192x2228x5840 539 / 433, but 11008x2560x1024, whole lines, 401 /
+    // 472), and so does one workgroup per CU on operands that no L2 holds (7392x72x2912 73 / 50,
+    // 37x13728x1992 53 / 41; 512x1536x768, in L2, 16.5 / 20).
+    if (vi.split == SplitKind::kPartial && splits == 1 && vi.vec) {
+        if (o.part_lines) cu_rate *= kWholePartLines;
+        if (per_cu == 1 && eb * (m * k + k * n) > kL2Bytes) cu_rate *= kWholeStreaming;
+    }
     const double rounds    = double(ceilDiv(per_cu, uint64_t(vi.occupancy)));
     // The deep-k kernel runs one workgroup per CU: each round pays the ramp
     // and, when split, its workgroups' partial-tile stores and arrival.
@@ -350,7 +364,11 @@ std::vector<std::string> ShapeCostFinder::candidates(const GemmProblem& problem,
     const int cus     = gemm::computeUnits(constraints.device());
     const bool has_c  = problem.c().memory() != nullptr;
     gemm::OperandForm o;
-    if (runs) o.tb = g.tb;
+    if (runs) {
+        const int64_t line = problem.a().numericType() == FTRAIN_NUMERIC_TYPE_FP32 ? 32 : 64;  // elements
+        o.tb               = g.tb;
+        o.part_lines       = g.lda % line != 0 || g.ldb % line != 0;
+    }
     std::vector<std::pair<double, int>> ranked;
     for (int i = 0; i < static_cast<int>(gemm::Variant::kCount); ++i) {
         // Only variants for a's element type compete.

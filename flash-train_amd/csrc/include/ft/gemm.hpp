@@ -127,7 +127,8 @@ void forceSplits(uint32_t s);
 
 // What the cost model takes of a problem's operands beside their sizes.
 struct OperandForm {
-    bool tb = false;  // column-major b
+    bool tb         = false;  // column-major b
+    bool part_lines = false;  // rows (leading dimension) of a or b not whole 128-byte lines
 };
 
 // Modelled execution time in microseconds (lower is better).

@@ -610,6 +610,17 @@ def test_finder_choices_for_the_baseline_configs(tlib):
     # 1024^3: DMA 64x128 split-k 25.7, the deep-k tile unsplit 26.7, DMA 128x64 split-k 27.9.
     assert rank(tlib, 1024, 1024, 1024)[0] in ("Fp32Mfma16Gemm_64x64_DeepK", "Fp32Mfma16Gemm_64x128_Dma_SplitK",
                                                "Fp32Mfma16Gemm_64x64_Dma_SplitK")
+    # The 64x64 split tile's whole-k form: kept where the rows are whole lines (11008x2560x1024 401 against 472 for
+    # the 128x128 tile, 512x1536x768 16.5 against 20), not on rows of part lines (3652x12080x7296 4764 against 4411,
+    # 9584x4124x7564 4380 against 4177) nor for one workgroup per CU on large operands (7392x72x2912 73 against 50).
+    names = {tlib.ftrainTestingVariantName(i).decode(): i for i in range(tlib.ftrainTestingVariantCount())}
+
+    def whole64(m, n, k, tb=False):
+        first = rank(tlib, m, n, k, tb=tb)[0]
+        return first == "Fp32Mfma16Gemm_64x64_Dma_SplitK" and tlib.ftrainTestingChooseSplits(names[first], m, n, k, 256) == 1
+
+    assert whole64(11008, 2560, 1024) and whole64(512, 1536, 768)
+    assert not whole64(3652, 12080, 7296) and not whole64(9584, 4124, 7564) and not whole64(7392, 72, 2912, tb=True)
     # GEMV: the one-pass kernel (37.8 us) against split-k plus its reduction (47.6 us).
     assert rank(tlib, 1, 8192, 8192)[0] == "Fp32Gemv"
     # It also wins with 128 (1x4096x8192: 24.8 against 39.2 us) and 64 workgroups of 16 waves
