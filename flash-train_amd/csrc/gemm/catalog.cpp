@@ -77,11 +77,11 @@ constexpr VariantInfo kInfo[] = {
     {"Bf16MfmaGemm_256x256", 256, 256, 64, 512, 1, true, N, false, false, true, 0.6, BF16, 4096.0, 0.6},
     {"Bf16MfmaGemm_128x128", 128, 128, 64, 256, 2, true, N, false, false, true, 0.4, BF16, 4096.0, 0.4},
     {"Bf16MfmaGemm_128x128_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.42, BF16, 4096.0, 0.3},
-    {"Bf16MfmaGemm_64x64_Unaligned", 64, 64, 32, 256, 2, false, N, false, false, true, 0.08, BF16, 4096.0, 0.08},
+    {"Bf16MfmaGemm_64x64_Unaligned", 64, 64, 32, 256, 2, false, N, false, false, true, 0.08, BF16, 4096.0, 0.03},
     {"Fp16MfmaGemm_256x256", 256, 256, 64, 512, 1, true, N, false, false, true, 0.6, FP16, 4096.0, 0.6},
     {"Fp16MfmaGemm_128x128", 128, 128, 64, 256, 2, true, N, false, false, true, 0.4, FP16, 4096.0, 0.4},
     {"Fp16MfmaGemm_128x128_SplitK", 128, 128, 64, 256, 2, true, P, false, false, true, 0.42, FP16, 4096.0, 0.3},
-    {"Fp16MfmaGemm_64x64_Unaligned", 64, 64, 32, 256, 2, false, N, false, false, true, 0.08, FP16, 4096.0, 0.08},
+    {"Fp16MfmaGemm_64x64_Unaligned", 64, 64, 32, 256, 2, false, N, false, false, true, 0.08, FP16, 4096.0, 0.03},
     {"Bf16MfmaGemm_256x256_Dma", 256, 256, 64, 512, 1, true, N, false, false, true, 0.80, BF16, 4096.0, 0.80},
     {"Fp16MfmaGemm_256x256_Dma", 256, 256, 64, 512, 1, true, N, false, false, true, 0.80, FP16, 4096.0, 0.80},
     {"Bf16MfmaGemm_128x128_Dma", 128, 128, 64, 256, 2, true, N, false, false, true, 0.48, BF16, 4096.0, 0.60},

@@ -64,6 +64,10 @@ constexpr double kTieWeight       = 1e-3;
 constexpr double kWholePartLines = 0.95;
 constexpr double kWholeStreaming = 0.72;
 constexpr double kL2Bytes        = 32.0 * 1048576.0;
+// Whole-k 16-bit tiles on few workgroups, see modelMicros: MFMA time on rows of part lines, and a 16-bit c
+// on a 128-row tile.
+constexpr double kHalfPartLines = 1.4;
+constexpr double kHalfCMicros   = 9.0;
 // The skinny kernel for a column-major b with five rows or more: bytes per microsecond over its rounds of
 // one workgroup per CU, and a fixed cost.
 constexpr double kGemvManyRowsRate   = 5.6e6;
@@ -86,6 +90,10 @@ uint64_t ceilDiv(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 // The 16-bit 64x128 split tile (m of at most 64).
 bool half64x128(const VariantInfo& vi) {
     return vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 64 && vi.bn == 128 && vi.split == SplitKind::kPartial;
+}
+
+bool half128Dma(const VariantInfo& vi) {
+    return vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 128 && std::strstr(vi.name, "_Dma") != nullptr;
 }
 
 bool half256Dma(const VariantInfo& vi) {
@@ -214,8 +222,7 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
     // The 16-bit 128x128 DMA tiles between one and two workgroups per CU: a second workgroup costs a
     // CU half of what the first does, and only some CUs hold one (bf16, k 4096: 288 tiles 45 us, 384 52,
     // 512 60).
-    if (vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 128 && std::strstr(vi.name, "_Dma") != nullptr &&
-        wgs > uint64_t(cus) && wgs <= 2 * uint64_t(cus)) {
+    if (half128Dma(vi) && wgs > uint64_t(cus) && wgs <= 2 * uint64_t(cus)) {
         const double one = mfma / 2.0 * residentEfficiency(vi, 2) / kPairedSoloEfficiency;
         mfma             = one + (mfma - one) * (double(wgs) / double(cus) - 1.0);
     }
@@ -227,6 +234,17 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
     if (vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.bm == 256 && s.n % 32 == 0 && wgs > uint64_t(cus) &&
         5 * wgs <= 6 * uint64_t(cus))
         mfma += kThinRoundMicros;
+    // Whole-k 16-bit tiles other than the 256x256 DMA one, where a split over k would still be one round.
+    // Rows of part lines slow a 128x128 tile's loads (bf16, us, whole-k against split 128x128 DMA tile:
+    // 141x1176x1128 14.2 / 9.4, 253x2136x1392 16.6 / 13.1, 233x3336x1560 18.5 / 14.8; whole lines 350x1824x1088
+    // 10.5 / 11.6), and a 16-bit c, which these tiles load 2 bytes at a time, comes on top (122x2032x1144 with c
+    // 21.6 / 11.0, 107x6680x1552 29.0 / 14.3, 659x1384x704 20.7 / 11.9).  The per-element 64x64 tile pays for
+    // its c at any number of workgroups (596x2864x568 26.8 against 16.5 on the split tile).
+    if (vi.input != FTRAIN_NUMERIC_TYPE_FP32 && vi.split == SplitKind::kNone && !half256Dma(vi)) {
+        const bool few = 2 * wgs <= uint64_t(cus);
+        if (vi.bm == 128 && o.part_lines && few) mfma *= kHalfPartLines;
+        if (has_c && o.cd_half && (vi.bm == 64 || few)) mfma += kHalfCMicros * vi.bm / 128.0;
+    }
     const double compute   = mfma + rounds * per_round + tails * kDmaTailMicros * std::min(1.0, vi.bm * vi.bn / 65536.0);
     // A launch with fewer workgroups than CUs streams memory through only that many of them (a CU
     // moves a bounded number of bytes per clock): 64x4096x14336 bf16 on the 64x128 split tile took
@@ -313,7 +331,10 @@ uint32_t chooseSplits(Variant v, const GemmShape& s, int cus) {
         // Not for the 16-bit 64x128 tile: it streams from memory, and workgroups just past a multiple of
         // the CUs cost it more than the finer choice gives (bf16, column-major b, us at 2 / 3 / 4 splits:
         // 16x11008x5120 28.6 / 33.1 / 29.8, 4x13824x5120 30.6 / 35.2 / 32.6; 2x6016x8992 at 4 / 6 25.0 / 32.0).
-        if (!vi.gemv && !half64x128(vi) && sp + sp / 2 <= most) consider(sp + sp / 2);
+        // Nor for the 128x128 DMA tile where that one applies: a finer count would win it the tie on memory
+        // that the smaller tile runs faster (bf16, 64x128 / 128x128 tile: 42x13040x13920 87 / 110 at 3 splits,
+        // 12x12168x13472 60 / 81, 57x11832x6224 45 / 57).
+        if (!vi.gemv && !half64x128(vi) && !(half128Dma(vi) && s.m <= 64) && sp + sp / 2 <= most) consider(sp + sp / 2);
     }
     return static_cast<uint32_t>(best);
 }
@@ -367,6 +388,7 @@ std::vector<std::string> ShapeCostFinder::candidates(const GemmProblem& problem,
     if (runs) {
         const int64_t line = problem.a().numericType() == FTRAIN_NUMERIC_TYPE_FP32 ? 32 : 64;  // elements
         o.tb               = g.tb;
+        o.cd_half          = problem.d().numericType() != FTRAIN_NUMERIC_TYPE_FP32;
         o.part_lines       = g.lda % line != 0 || g.ldb % line != 0;
     }
     std::vector<std::pair<double, int>> ranked;

@@ -128,6 +128,7 @@ void forceSplits(uint32_t s);
 // What the cost model takes of a problem's operands beside their sizes.
 struct OperandForm {
     bool tb         = false;  // column-major b
+    bool cd_half    = false;  // 16-bit c and d
     bool part_lines = false;  // rows (leading dimension) of a or b not whole 128-byte lines
 };
 

@@ -706,6 +706,17 @@ def test_finder_choices_for_16_bit_tiles(tlib):
     assert rank(tlib, 8192, 8192, 8200, ab_type=c.BF16)[0] == "Bf16MfmaGemm_256x256_Dma"
     assert rank(tlib, 16384, 14336, 4104, ab_type=c.BF16)[0] == "Bf16MfmaGemm_256x256_Dma"
     assert rank(tlib, 4096, 4096, 4100, ab_type=c.BF16) == ["Bf16MfmaGemm_64x64_Unaligned"]
+    # A wide n over a deep k streams from memory: the 64x128 tile, not the 128x128 one at 3 * 2^i splits (bf16, us:
+    # 87 against 110, 60 against 81).
+    assert rank(tlib, 42, 13040, 13920, ab_type=c.BF16, tb=True)[0] == tile64
+    assert rank(tlib, 12, 12168, 13472, ab_type=c.BF16, cd_type=c.BF16)[0] == tile64
+    # Few whole-k 128x128 workgroups lose to split ones on rows of part lines (14.2 against 9.4, 18.5 against 14.8) and
+    # with a 16-bit c (21.6 against 11.0, 29.0 against 14.3, 20.7 against 11.9).
+    split = "Bf16MfmaGemm_128x128_Dma_SplitK"
+    assert rank(tlib, 141, 1176, 1128, ab_type=c.BF16, cd_type=c.BF16)[0] == split
+    assert rank(tlib, 233, 3336, 1560, ab_type=c.BF16, cd_type=c.BF16)[0] == split
+    for shape in ((122, 2032, 1144), (107, 6680, 1552), (659, 1384, 704)):
+        assert rank(tlib, *shape, ab_type=c.BF16, cd_type=c.BF16, with_c=True, tb=True)[0] == split, shape
     # Taller problems keep the 128-row tiles: the 64-row one does not apply above m = 64.
     assert tile64 not in rank(tlib, 65, 4096, 4096, ab_type=c.BF16)
     assert "Fp16MfmaGemm_64x128_Dma_SplitK" == rank(tlib, 64, 4096, 4096, ab_type=c.FP16)[0]
