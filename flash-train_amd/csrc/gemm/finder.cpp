@@ -55,9 +55,6 @@ constexpr double kFusedStoreMicros    = 2.0;  // per round: a split workgroup's 
 // stores, the ramp of the first stages); fitted with the catalog efficiencies.
 constexpr double kRoundMicros     = 3.35;
 constexpr double kThinRoundMicros = 7.0;  // a second round on few CUs, see modelMicros
-// The 16-bit 256x256 DMA tile's sustained fraction in a grouped launch, which reads every group's own
-// weight from memory (MLP forward over 8 experts 0.53 of peak, plain 0.58-0.62).
-constexpr double kGroupedHalf256Efficiency = 0.66;
 constexpr double kTieWeight       = 1e-3;
 // The whole-k form of the fp32 64x64 split tile, see modelMicros: its rate on rows of part lines, and of one
 // workgroup per CU on operands larger than the L2s (8 of 4 MiB).
@@ -74,11 +71,9 @@ constexpr double kGemvManyRowsRate   = 5.6e6;
 constexpr double kGemvManyRowsMicros = 2.0;
 constexpr double kCuBytesPerMicro = 6.4e4;  // one CU's sustained load rate (about 27 bytes per clock)
 // A DMA tile stages a partial last stage (k not a multiple of its stage) by ordinary loads once its
-// pipeline has drained: per tile, the drain, the loads' latency and a barrier.  Fitted to the bf16
-// grouped weight gradient (16384 ragged tokens, 4096x14336 weights, ms, DMA against register-staged
-// 256x256 tile): 8 experts 1.80 / 2.01, 16 2.25 / 2.42, 32 3.28 / 3.23, 64 5.28 / 4.86, 128 9.15 /
-// 8.22; the DMA tile is ranked first at 8 experts only (7% lost at 16).  A smaller tile stages as
-// much less: fp32 127x97x33 (one stage and a tail) takes 4.4 us in all on the 64x64 tile.
+// pipeline has drained: per tile, the drain, the loads' latency and a barrier (bf16 8192x8192x8200 819 us
+// on the 256x256 tile).  A smaller tile stages as much less: fp32 127x97x33 (one stage and a tail) takes
+// 4.6 us in all on the 64x64 tile.  Grouped 16-bit launches have their own figures (groupedTerms).
 constexpr double kDmaTailMicros = 3.0;  // of a 256x256 tile
 // Rate of a lone workgroup of the 16-bit 128x128 DMA tiles in their form for two per CU.
 constexpr double kPairedSoloEfficiency = 0.37;
@@ -101,10 +96,10 @@ bool half256Dma(const VariantInfo& vi) {
 }
 
 // Rows of a problem in tile rows of vi.  The 16-bit 256x256 DMA tile runs a last tile row of at most
-// 128 rows at half the cost.
+// 128 rows with half the MFMAs, in 70% of the time beside other tiles (fitted with groupedTerms).
 double tileRows(const VariantInfo& vi, uint64_t m) {
     const uint64_t rows = ceilDiv(m, vi.bm), left = m - (rows ? rows - 1 : 0) * vi.bm;
-    return half256Dma(vi) && left <= 128 ? double(rows) - 0.5 : double(rows);
+    return half256Dma(vi) && left <= 128 ? double(rows) - 0.3 : double(rows);
 }
 
 // Whether variant vi runs a k tail through the separate pass of the DMA tiles (stages of 32 k for
@@ -112,6 +107,8 @@ double tileRows(const VariantInfo& vi, uint64_t m) {
 bool dmaTail(const VariantInfo& vi, uint64_t k) {
     return std::strstr(vi.name, "_Dma") != nullptr && k % (vi.input == FTRAIN_NUMERIC_TYPE_FP32 ? 32 : 64) != 0;
 }
+
+double tailMicros(const VariantInfo& vi) { return kDmaTailMicros * std::min(1.0, vi.bm * vi.bn / 65536.0); }
 }  // namespace
 
 int computeUnits(FTrainDeviceId device) {
@@ -245,7 +242,7 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
         if (vi.bm == 128 && o.part_lines && few) mfma *= kHalfPartLines;
         if (has_c && o.cd_half && (vi.bm == 64 || few)) mfma += kHalfCMicros * vi.bm / 128.0;
     }
-    const double compute   = mfma + rounds * per_round + tails * kDmaTailMicros * std::min(1.0, vi.bm * vi.bn / 65536.0);
+    const double compute   = mfma + rounds * per_round + tails * tailMicros(vi);
     // A launch with fewer workgroups than CUs streams memory through only that many of them (a CU
     // moves a bounded number of bytes per clock): 64x4096x14336 bf16 on the 64x128 split tile took
     // 36.3 us at 4 splits (128 workgroups) against 23.8 us at 8.  On the 16-bit 64x128 split tile
@@ -347,32 +344,64 @@ double estimateMicros(Variant v, const GemmShape& s, bool has_c, int cus, const 
     return modelMicros(vi, s, has_c, cus, splits, o);
 }
 
-double groupedMicros(Variant v, const std::vector<GemmShape>& shapes, bool has_c, int cus) {
+namespace {
+// Terms of a grouped launch on a 16-bit tile, added up, in microseconds: per microsecond of MFMAs at peak rate
+// (padding included) of the CU with the most tiles, where it has one (alone) or more, and of all CUs on average
+// (mean: tiles of unlike depth even out); fixed; per round with a k tail; and per microsecond that the operands,
+// d, and a d whose rows are not whole 64-byte pieces take at HBM rate.  Unlike a plain launch, where the larger
+// of compute and memory decides, every group streams operands of its own through few workgroups.
+struct GroupedTerms {
+    double mfma, alone, mean, fixed, tail, operands, d, d_pieces;
+};
+
+// Fitted (least relative squares, MI355X) to every tile on 1197 sampled bf16 and fp16 products: 2 to 128 experts,
+// 32 to 32768 ragged tokens, sides of 64 to 14336, forward and weight gradient.  The tile ranked first takes 2%
+// longer than the fastest on average, also of those below 20 GFLOP; ranked by the terms of a plain launch it took
+// 6% longer in the large forwards, 26% in the large weight gradients and 17% in the small products (bf16, us,
+// register-staged / two-group 256x256 tile: weight gradient 5824x5736 over 53 experts and 1121 tokens 3888 /
+// 1623, 9584x4416 over 11 and 14374 1559 / 1215; forward, 128x128 DMA / two-group tile: 3805x10000x5776 over 9
+// experts 729 / 514, 1689x2136x3264 over 18 61 / 94).
+GroupedTerms groupedTerms(const VariantInfo& vi) {
+    const bool dma = std::strstr(vi.name, "_Dma") != nullptr;
+    if (vi.bm == 256)
+        return dma ? GroupedTerms{0.83, 1.17, 0.86, 4.0, 2.7, 0.59, 1.10, 0.20} : GroupedTerms{1.29, 1.41, 0.80, 4.6, 3.8, 0.32, 0.82, 1.25};
+    if (vi.bm == 128)
+        return dma ? GroupedTerms{2.22, 3.10, 0.28, 1.6, 2.0, 0.67, 0.70, 1.15} : GroupedTerms{2.61, 3.61, 0.29, 2.2, 2.5, 0.52, 0.72, 0.96};
+    return GroupedTerms{14.0, 30.6, 0.0, 2.3, 0.1, 0.0, 0.43, 0.41};
+}
+}  // namespace
+
+double groupedMicros(Variant v, const std::vector<GemmShape>& shapes, bool has_c, bool cd_half, int cus) {
     // The groups' tiles share one grid: a CU's load is its share of all
     // tiles, each costing its own group's depth; bytes add over the groups.
     const VariantInfo& vi = info(v);
-    const double eb = vi.input == FTRAIN_NUMERIC_TYPE_FP32 ? 4.0 : 2.0;
-    double flops = 0.0, bytes = 0.0;
+    const bool half = vi.input != FTRAIN_NUMERIC_TYPE_FP32;
+    const double eb = half ? 2.0 : 4.0, ed = cd_half ? 2.0 : 4.0;
+    double flops = 0.0, operands = 0.0, d = 0.0, d_pieces = 0.0;
     uint64_t tiles = 0, tail_tiles = 0;
     for (const GemmShape& s : shapes) {
         const uint64_t t = ceilDiv(s.m, vi.bm) * ceilDiv(s.n, vi.bn);
         tiles += t;
-        if (dmaTail(vi, s.k)) tail_tiles += t;
-        // A tile with a k tail gains less from a short last row (3143 tokens over 7 experts, 5984 columns,
-        // k 1040: 256x256 DMA tile 86 us, register-staged 78).
-        const double rows = dmaTail(vi, s.k) ? double(ceilDiv(s.m, vi.bm)) : tileRows(vi, s.m);
-        flops += rows * double(ceilDiv(s.n, vi.bn)) * 2.0 * vi.bm * vi.bn * double(std::max<uint64_t>(s.k, vi.bk));
-        bytes += eb * (double(s.m) * s.k + double(s.k) * s.n + double(s.m) * s.n * (has_c ? 2.0 : 1.0));
+        if (half ? s.k % 64 != 0 : dmaTail(vi, s.k)) tail_tiles += t;
+        flops += tileRows(vi, s.m) * double(ceilDiv(s.n, vi.bn)) * 2.0 * vi.bm * vi.bn * double(std::max<uint64_t>(s.k, half ? 64 : vi.bk));
+        operands += eb * (double(s.m) * s.k + double(s.k) * s.n);
+        const double out = ed * double(s.m) * double(s.n) * (has_c ? 2.0 : 1.0);
+        d += out;
+        if (s.n % (cd_half ? 32 : 16) != 0) d_pieces += out;
     }
     if (tiles == 0) return kLaunchMicros;
     const uint64_t per_cu = ceilDiv(tiles, cus);
-    const double cu_rate  = vi.flop_per_clk * kClockPerMicro *
-                            (half256Dma(vi) ? kGroupedHalf256Efficiency : residentEfficiency(vi, per_cu));
+    const double peak     = double(per_cu) * (flops / double(tiles)) / (vi.flop_per_clk * kClockPerMicro);
     const double rounds   = double(ceilDiv(per_cu, uint64_t(vi.occupancy)));
     const double tails    = double(ceilDiv(ceilDiv(tail_tiles, cus), uint64_t(vi.occupancy)));
-    const double compute  = double(per_cu) * (flops / double(tiles)) / cu_rate + rounds * kRoundMicros +
-                           tails * kDmaTailMicros;
-    return std::max(compute, bytes / kHbmBytesPerMicro) + kLaunchMicros;
+    if (half) {
+        const GroupedTerms g = groupedTerms(vi);
+        const double mean    = flops / (double(cus) * vi.flop_per_clk * kClockPerMicro);
+        return (per_cu > 1 ? g.mfma : g.alone) * peak + g.mean * mean + g.fixed + g.tail * tails +
+               (g.operands * operands + g.d * d + g.d_pieces * d_pieces) / kHbmBytesPerMicro + kLaunchMicros;
+    }
+    const double compute = peak / residentEfficiency(vi, per_cu) + rounds * kRoundMicros + tails * tailMicros(vi);
+    return std::max(compute, (operands + d) / kHbmBytesPerMicro) + kLaunchMicros;
 }
 
 }  // namespace gemm

@@ -564,10 +564,11 @@ std::vector<std::string> GroupedCostFinder::candidates(const GroupedGemmProblem&
         shapes.push_back(l.shape);
         has_c = has_c || l.c != nullptr;
     }
-    const int cus = gemm::computeUnits(constraints.device());
+    const int cus      = gemm::computeUnits(constraints.device());
+    const bool cd_half = problem.d().type != FTRAIN_NUMERIC_TYPE_FP32;
     std::vector<std::pair<double, const char*>> ranked;
     for (const GroupedVariant& v : kGroupedVariants)
-        if (v.input == problem.a().type) ranked.emplace_back(gemm::groupedMicros(v.tile, shapes, has_c, cus), v.name);
+        if (v.input == problem.a().type) ranked.emplace_back(gemm::groupedMicros(v.tile, shapes, has_c, cd_half, cus), v.name);
     std::stable_sort(ranked.begin(), ranked.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
     std::vector<std::string> names;
     for (const auto& r : ranked) names.emplace_back(r.second);

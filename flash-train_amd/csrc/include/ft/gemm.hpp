@@ -139,8 +139,8 @@ double estimateMicros(Variant v, const GemmShape& s, bool has_c, int cus, const 
 int computeUnits(FTrainDeviceId device);
 
 // Modelled microseconds of one grouped launch over the groups' (kernel-
-// orientation) shapes with tile variant v.
-double groupedMicros(Variant v, const std::vector<GemmShape>& shapes, bool has_c, int cus);
+// orientation) shapes with tile variant v; cd_half: c and d are 16-bit.
+double groupedMicros(Variant v, const std::vector<GemmShape>& shapes, bool has_c, bool cd_half, int cus);
 
 }  // namespace gemm
 

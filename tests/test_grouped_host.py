@@ -10,6 +10,7 @@ fake device addresses (never dereferenced before execution).
 """
 
 import ctypes
+import math
 
 import pytest
 
@@ -84,6 +85,61 @@ def test_large_groups_take_the_large_tiles(tlib):
     st, msg, plan = moe_abcd(tlib, rows, k=4096, n=14336, a_type=c.BF16)
     assert st == c.SUCCESS, msg
     assert plan.names()[0] == "GroupedBf16MfmaGemm_256x256_Dma"
+
+
+def uneven(total, groups):
+    """Token counts between 0.4 and 1.6 times their mean, adding up to the total."""
+    weights = [1.0 + 0.6 * math.sin(1.7 * g + 0.3) for g in range(groups)]
+    counts = [int(total * w / sum(weights)) for w in weights]
+    counts[-1] += total - sum(counts)
+    return counts
+
+
+def weight_gradient(tlib, tokens, m, n, ab_type=c.BF16):
+    G, total = len(tokens), sum(tokens)
+    first = [sum(tokens[:g]) for g in range(G)]
+    al, be = c.HostScalar(1.0), c.HostScalar(0.0)
+    args = c.GroupedOps("ab", l=tlib).args(
+        a=c.GroupedSpec(D([total, m], numeric_type=ab_type), G, dims=[(m, t) for t in tokens], strides=[(1, m)] * G,
+                        offsets=[f * m for f in first]),
+        b=c.GroupedSpec(D([total, n], numeric_type=ab_type), G, dims=[(t, n) for t in tokens]),
+        c=[D([m, n], None) for _ in tokens], d=[D([m, n]) for _ in tokens], alpha=al.view, beta=be.view)
+    st, msg, plan = args.plan_status_on_device(0)
+    assert st == c.SUCCESS, msg
+    return plan.names()[0]
+
+
+def test_ragged_16_bit_weight_gradients_take_the_faster_tile(tlib):
+    # us on MI355X: register-staged 256x256, two-group 256x256, 128x128 DMA (every k has a tail).
+    for m, n, total, groups, staged, two_group, small in (
+            (4096, 14336, 16384, 8, 2060, 1638, 2202), (5824, 5736, 1121, 53, 3888, 1623, 2672), (8912, 7256, 2098, 30, 4253, 1936, 3845),
+            (9584, 4416, 14374, 11, 1559, 1215, 1474), (4600, 8872, 1114, 4, 379, 225, 359),
+            (3984, 3856, 15622, 63, 1296, 1392, 1159), (12760, 1648, 3465, 43, 828, 1025, 799)):
+        first = weight_gradient(tlib, uneven(total, groups), m, n)
+        fastest = min((staged, "GroupedBf16MfmaGemm_256x256"), (two_group, "GroupedBf16MfmaGemm_256x256_Dma"),
+                      (small, "GroupedBf16MfmaGemm_128x128_Dma"))[1]
+        assert first == fastest, (m, n, total, groups, first)
+
+
+def test_16_bit_forwards_take_the_faster_tile(tlib):
+    # us on MI355X: two-group 256x256, 128x128 DMA, register-staged 256x256, per-element 64x64; few tokens and small sides
+    # included.
+    for rows, n, k, groups, d_type, two_group, small, staged, tiny in (
+            (16384, 14336, 4096, 64, c.FP32, 2310, 2710, 2903, 8939), (3805, 10000, 5776, 9, c.BF16, 514, 729, 691, 2407),
+            (8461, 3288, 1064, 10, c.BF16, 85, 106, 127, 319), (1689, 2136, 3264, 18, c.FP32, 94, 61, 140, 139),
+            (184, 104, 1640, 3, c.BF16, 24, 21, 43, 52), (208, 1768, 1200, 2, c.BF16, 21, 19, 36, 41)):
+        al, be = c.HostScalar(1.0), c.HostScalar(0.0)
+        counts = uneven(rows, groups)
+        args = c.GroupedOps("abcd", l=tlib).args(
+            a=c.GroupedSpec(D([rows, k], numeric_type=c.BF16), groups, dims=[(r, k) for r in counts]),
+            b=c.GroupedSpec(D([k, n], numeric_type=c.BF16), groups),
+            c=c.GroupedSpec(D([rows, n], None, numeric_type=d_type), groups, dims=[(r, n) for r in counts]),
+            d=c.GroupedSpec(D([rows, n], numeric_type=d_type), groups, dims=[(r, n) for r in counts]), alpha=al.view, beta=be.view)
+        st, msg, plan = args.plan_status_on_device(0)
+        assert st == c.SUCCESS, msg
+        fastest = min((two_group, "GroupedBf16MfmaGemm_256x256_Dma"), (small, "GroupedBf16MfmaGemm_128x128_Dma"),
+                      (staged, "GroupedBf16MfmaGemm_256x256"), (tiny, "GroupedBf16MfmaGemm_64x64_Unaligned"))[1]
+        assert plan.names()[0] == fastest, (rows, n, k, groups, plan.names())
 
 
 def test_disabled_grouped_finder_falls_back_to_registration_order():
