@@ -73,6 +73,11 @@ FTRAIN_TESTING_API uint32_t ftrainTestingChooseSplits(int v, uint64_t m, uint64_
     return gemm::chooseSplits(static_cast<gemm::Variant>(v), GemmShape{m, n, k}, cus);
 }
 
+FTRAIN_TESTING_API bool ftrainTestingTakes128(uint64_t m, uint64_t n, uint64_t k, bool ta, bool tb, bool has_c,
+                                              bool cd_half, int cus) {
+    return gemm::takes128(GemmShape{m, n, k}, ta, tb, has_c, cd_half, cus);
+}
+
 FTRAIN_TESTING_API void ftrainTestingForceSplits(uint32_t s) { gemm::forceSplits(s); }
 
 // Convenience Plans still alive (cached per thread or owned by captured graphs).

@@ -344,6 +344,24 @@ double estimateMicros(Variant v, const GemmShape& s, bool has_c, int cus, const 
     return modelMicros(vi, s, has_c, cus, splits, o);
 }
 
+// A row-major b needs n, a column-major a m of at least a tile (the kernel moves its last tile inside the
+// matrix).  The large tile runs a stage in half the time, but costs more before its first and after its last
+// one, most with a 16-bit c, which it loads 2 bytes at a time.  bf16, us, 64x64 / 128x128 tile:
+//   16-bit c and d: 1000x1003x700 28 / 36, x1100 40 / 40; 1500x3501x316 36 / 37, x700 60 / 45; 3000x4001x700
+//     100 / 80; column-major b 1000x3003x700 31 / 36, x1100 44 / 42, 4000x9001x316 131 / 171, x700 224 / 204;
+//   fp32 c and d: 1000x1003x508 20 / 22, x700 26 / 24, x1100 37 / 28; 3000x4001x316 55 / 58, x508 75 / 64;
+//     column-major b 3000x4001x508 64 / 63, 4000x9001x508 174 / 174, x1100 330 / 211;
+//   no c: 1000x1003x316 12 / 13, x508 18 / 15, x700 24 / 16; 3000x4001x316 46 / 48, x508 66 / 53; column-major b
+//     1000x1003x508 16 / 16, x700 21 / 18; 4000x9001x316 111 / 134, x508 158 / 143; 16-bit d 1000x1003x316
+//     13 / 18, x700 25 / 21.
+bool takes128(const GemmShape& s, bool ta, bool tb, bool has_c, bool cd_half, int cus) {
+    if (s.m <= 64 || s.n <= 64 || (ta && s.m < 128) || (!tb && s.n < 128)) return false;
+    const uint64_t tiles = ceilDiv(s.m, 64) * ceilDiv(s.n, 64);
+    if (has_c && cd_half) return s.k >= (tiles > 4 * uint64_t(cus) ? 640 : 1152);
+    if (tiles > 2 * uint64_t(cus)) return s.k >= (tb || has_c ? 512 : 384);
+    return s.k >= 640;
+}
+
 namespace {
 // Terms of a grouped launch on a 16-bit tile, added up, in microseconds: per microsecond of MFMAs at peak rate
 // (padding included) of the CU with the most tiles, where it has one (alone) or more, and of all CUs on average

@@ -89,21 +89,6 @@ bool fits128(const GemmProblem& p, const GemmLaunch& g) {
     return true;
 }
 
-// Whether the 16-bit per-element variant runs a problem on its 128x128 tile (16-byte loads at any
-// address).  A row-major b needs n, a column-major a m of at least a tile (the kernel moves its last
-// tile inside the matrix).  The large tile costs more before its first and after its last stage (most
-// with a c to read), so a short k stays on the small one: bf16, us, per-element tile against it, row-major
-// b without c: 1000x1003x316 12.3 / 16.2, x700 23.3 / 20.1, x2044 62 / 32; 500x3001x444 17.4 / 17.5;
-// 1000x3003x316 16.2 / 16.7, x444 20.6 / 18.1; 1000x5003x2048 87 / 41.  Column-major b with c: 278x3201x316
-// 12.3 / 21.0, x700 25.3 / 30.9, x1100 36.4 / 36.5, x2044 59 / 43; 1000x3003x700 30.9 / 34.9, x1100 43 / 39.
-bool takes128(const GemmLaunch& g) {
-    const GemmShape s = g.shape;
-    if (s.m <= 64 || s.n <= 64 || (g.ta && s.m < 128) || (!g.tb && s.n < 128)) return false;
-    const uint64_t tiles = ceilDiv(s.m, 64) * ceilDiv(s.n, 64);
-    if (g.tb || g.c != nullptr) return s.k >= 1152;
-    return s.k >= (tiles > 512 ? 384 : 640);
-}
-
 // The launch's workgroup size must equal the kernel's launch bounds (every
 // kernel here declares its exact size: a larger launch fails, a smaller one
 // would leave part of each tile uncomputed).  Checked when HIP can describe
@@ -292,7 +277,7 @@ class GemmPrimitive final : public Primitive<GemmProblem> {
             params_.tiles_n = half_params_.tiles_n = int32_t(ceilDiv(s.n, info_->bn));
             grid_           = dim3(uint32_t(params_.tiles_m) * uint32_t(params_.tiles_n), 1, splits);
             const bool per_element = v_ == Variant::kBf16Mfma64x64U || v_ == Variant::kFp16Mfma64x64U;
-            if (per_element && takes128(g)) {
+            if (per_element && gemm::takes128(s, g.ta, g.tb, g.c != nullptr, cd_half, cus)) {
                 half_params_.tiles_m = int32_t(ceilDiv(s.m, 128));
                 half_params_.tiles_n = int32_t(ceilDiv(s.n, 128));
                 grid_   = dim3(uint32_t(half_params_.tiles_m) * uint32_t(half_params_.tiles_n));

@@ -135,6 +135,10 @@ struct OperandForm {
 // Modelled execution time in microseconds (lower is better).
 double estimateMicros(Variant v, const GemmShape& s, bool has_c, int cus, const OperandForm& o = {});
 
+// Whether a 16-bit per-element variant runs a problem on its 128x128 tile (16-byte loads at any address)
+// instead of its 64x64 one; cd_half: c and d are 16-bit.
+bool takes128(const GemmShape& s, bool ta, bool tb, bool has_c, bool cd_half, int cus);
+
 // Compute units of `device` (cached; 256 when HIP cannot be queried).
 int computeUnits(FTrainDeviceId device);
 

@@ -722,6 +722,25 @@ def test_finder_choices_for_16_bit_tiles(tlib):
     assert "Fp16MfmaGemm_64x128_Dma_SplitK" == rank(tlib, 64, 4096, 4096, ab_type=c.FP16)[0]
 
 
+def test_unaligned_16_bit_products_take_the_faster_tile(tlib):
+    # bf16, us: (m, n, k, column-major b, c, 16-bit c and d, 64x64 tile, 128x128 tile).
+    for m, n, k, tb, with_c, half, small, large in (
+            (4000, 9001, 1100, False, True, False, 386, 213), (4000, 9001, 1100, True, False, False, 318, 185),
+            (4000, 9001, 700, False, True, True, 276, 196), (3000, 4001, 1100, False, True, False, 141, 86),
+            (3000, 4001, 700, True, False, False, 76, 59), (1500, 3501, 1100, True, True, False, 77, 42),
+            (1500, 3501, 700, True, True, True, 53, 46), (1000, 3003, 1100, True, False, False, 39, 24),
+            (526, 1575, 700, True, False, True, 22, 17), (500, 500, 700, False, True, False, 25, 23),
+            (1000, 1003, 2044, False, True, False, 63, 37), (1000, 5003, 2048, False, False, False, 87, 40),
+            (1000, 1003, 700, False, True, True, 28, 36), (1000, 3003, 700, True, True, True, 31, 36),
+            (1000, 1003, 316, False, False, False, 12, 13), (1000, 1003, 508, False, True, False, 20, 22),
+            (3000, 4001, 316, True, False, False, 42, 48), (4000, 9001, 316, True, True, True, 131, 171)):
+        assert tlib.ftrainTestingTakes128(m, n, k, False, tb, with_c, half, 256) == (large < small), (m, n, k, tb, with_c, half)
+    # A whole tile has to exist along a column-major a's rows and a row-major b's columns.
+    assert not tlib.ftrainTestingTakes128(127, 4000, 4000, True, True, False, False, 256)
+    assert not tlib.ftrainTestingTakes128(4000, 127, 4000, False, False, False, False, 256)
+    assert tlib.ftrainTestingTakes128(127, 127, 4000, False, True, False, False, 256)
+
+
 def test_finder_respects_alignment_and_row_limits(tlib):
     names = rank(tlib, 512, 512, 512, addr=FAKE + 4)
     assert names and all(("Unaligned" in n) or n == "Fp32Gemm" for n in names)

@@ -138,7 +138,8 @@ def test_half_256_tile_in_place(capi, ops):
 @pytest.mark.parametrize("m,n", [(128, 128), (2048, 2048), (2048, 2176)])
 def test_half_128_tile_stage_counts(capi, ops, m, n):
     for k in (40, 64, 128, 192, 200, 256, 320, 384, 456):
-        check(capi, ops, "bf16", "fp32", m, n, k, False, True, False, only="128x128_Dma")
+        names = check(capi, ops, "bf16", "fp32", m, n, k, False, True, False, only="128x128_Dma")
+        assert "Bf16MfmaGemm_128x128_Dma" in names, names
 
 
 # fp32 without 16-byte alignment: rows, columns and depths of every remainder by 4, one to several
@@ -175,6 +176,8 @@ def test_fp32_unaligned_in_place(capi, ops):
 @pytest.mark.parametrize("kind,cd", [("bf16", "fp32"), ("fp16", "fp16")])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 def test_half_unaligned_tiles(capi, ops, kind, cd, ta, tb):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    large = {}
     for m, n, k in ((129, 131, 1281), (128, 128, 1283), (255, 257, 1151), (255, 257, 1215), (300, 129, 1407),
                     (131, 300, 1344), (65, 66, 100), (127, 127, 1300), (66, 500, 1357), (300, 129, 639), (131, 300, 641),
                     (1500, 1601, 385)):
@@ -182,6 +185,11 @@ def test_half_unaligned_tiles(capi, ops, kind, cd, ta, tb):
             names = check(capi, ops, kind, cd, m, n, k, ta, tb, with_c, ab_pad, ab_shift, cd_pad, 1 if cd_pad else 0,
                           only="Unaligned")
             assert any("64x64_Unaligned" in nm for nm in names), names
+            large[m, n, k, with_c] = capi.testing_lib().ftrainTestingTakes128(m, n, k, ta, tb, with_c, cd != "fp32", cus)
+    # The Primitive ran both of its tiles, the 128x128 one with moved last tiles and shifted k-tail chunks among them.
+    assert all(large[m, n, k, with_c] for m, n, k in ((129, 131, 1281), (128, 128, 1283), (255, 257, 1215), (300, 129, 1407),
+                                                      (131, 300, 1344)) for with_c in (False, True)), large
+    assert not all(large.values()), large
 
 
 def test_half_unaligned_in_place(capi, ops):
