@@ -11,11 +11,13 @@
 // src/primitive/hygon/gemm/fp32_gemm.hip:18-31: the beta term dropped for a
 // null c, always evaluated otherwise); the split-k form writes each split's
 // raw partial tile to slice z of the workspace (dense m x n) and
-// splitk_reduce forms d.  Applicability, checked on the host: k a positive
-// multiple of 32, n a multiple of 4, 16-byte aligned a, b, c, d with leading
-// dimensions multiples of 4, a's and b's below 2^22 elements and c's and d's
-// below 2^21 (32-bit offsets); m and n are free otherwise (edge tiles clamp
-// their loads and drop their out-of-matrix stores).
+// splitk_reduce forms d.  Applicability, checked on the host: k positive,
+// leading dimensions of a and b below 2^22 elements and of c and d below 2^21
+// (32-bit offsets); the aligned forms also need n and the contiguous extents
+// of a and b multiples of 4 and 16-byte aligned a, b, c, d with leading
+// dimensions multiples of 4, the unaligned ones (U) a row-major a and n of at
+// least 4.  m, n and k are free otherwise (edge tiles clamp their loads and
+// drop their out-of-matrix stores; a k tail is staged by ordinary loads).
 //
 // Wave tile: TM x TN blocks of 16x16 outputs:
 //   A operand: lane l holds A[row l % 16][k slot g = l / 16]

@@ -125,8 +125,10 @@ enum class Variant : int {
     // v_mfma_f32_16x16x4_f32 256x256 tiles, 4 waves of 128x128 (one per
     // SIMD), 128-bit loads, every operand orientation; whole-k and split-k.
     // fp32 tiles with operands staged into LDS by DMA (global_load_lds_dwordx4),
-    // v_mfma_f32_16x16x4_f32: row-major a and b, k a multiple of 32, any m and
-    // n; 256x256 (one workgroup per CU) and 128x128 whole-k, and split-k forms.
+    // v_mfma_f32_16x16x4_f32: any m, n and k with rows of 16-byte units; row-major
+    // a and b on every tile, a column-major b on all but 256x256, a column-major a
+    // on some.  256x256 (one workgroup per CU) and smaller, whole-k and split-k;
+    // 64x64 split-k, which also runs whole-k as one split (unsplitForm).
     kMfma16Dma256x256,
     kMfma16Dma256x256S,
     kMfma16Dma128x128,
