@@ -67,8 +67,8 @@ constexpr double kHalfPartLines = 1.4;
 constexpr double kHalfCMicros   = 9.0;
 // The skinny kernel for a column-major b with five rows or more: bytes per microsecond over its rounds of
 // one workgroup per CU, and a fixed cost.
-constexpr double kGemvManyRowsRate   = 5.6e6;
-constexpr double kGemvManyRowsMicros = 2.0;
+constexpr double kGemvManyRowsRate   = 5.9e6;
+constexpr double kGemvManyRowsMicros = 9.0;
 constexpr double kCuBytesPerMicro = 6.4e4;  // one CU's sustained load rate (about 27 bytes per clock)
 // A DMA tile stages a partial last stage (k not a multiple of its stage) by ordinary loads once its
 // pipeline has drained: per tile, the drain, the loads' latency and a barrier (bf16 8192x8192x8200 819 us
@@ -174,7 +174,7 @@ double modelMicros(const VariantInfo& vi, const GemmShape& s, bool has_c, int cu
         // From five rows on, the form for a column-major b has room for one workgroup per CU: a last round
         // on few CUs takes as long as a full one (us, against the best split tile: 8x8192x8192, 256
         // workgroups, 58.7 / 74.9; 7x12768x4600, 399, 50 / 64; 5x8824x13680, 276, 183 / 127; 6x11688x12376,
-        // 366, 174 / 147; 5x9864x2488, 309, 41 / 34).
+        // 366, 174 / 147; 6x11440x6728, 358, 96 / 84; 8x9616x1416, 301, 27.6 / 23.2).
         if (o.tb && vi.split == SplitKind::kNone && s.m > 4)
             return std::ceil(wgs / double(cus)) * double(cus) / wgs * bytes / kGemvManyRowsRate + kGemvManyRowsMicros + launch;
         const double t      = std::max(bytes / (kHbmBytesPerMicro * fill), per_cu / kCuBytesPerMicro) + serial_us + launch;

@@ -652,7 +652,8 @@ def test_finder_choices_for_a_skinny_column_major_b(tlib):
     # with one or two rows, and with more only where its workgroups of 32 columns fill their rounds of the 256 CUs.
     for m, n, k, skinny, tile in ((1, 8192, 8192, 44.7, 73.2), (2, 6832, 2520, 13.5, 26.0), (4, 12304, 3064, 34.0, 48.6),
                                   (8, 8192, 8192, 58.7, 74.9), (7, 12768, 4600, 49.7, 66), (5, 8824, 13680, 183, 127),
-                                  (6, 11688, 12376, 174, 147), (5, 9476, 7912, 101, 81)):
+                                  (6, 11688, 12376, 174, 147), (5, 9476, 7912, 101, 81),
+                                  (6, 11440, 6728, 96, 84), (8, 9616, 1416, 27.6, 23.2), (7, 8672, 2040, 36, 28)):
         first = rank(tlib, m, n, k, tb=True)[0]
         assert (first == "Fp32Gemv") == (skinny < tile), (m, n, k, first)
 
